@@ -1,12 +1,14 @@
 // Causal attention forward (prefill) with native GQA and logsumexp output.
 //
-// Two kernels, chosen by dtype and head_dim:
+// Three kernels, chosen by dtype and head_dim:
 //   * prefill_mfma_kernel (bf16/f16, D a multiple of 8 up to 128): flash
 //     attention on v_mfma_f32_32x32x16_{bf16,f16} with K/V tiles
 //     double-buffered through LDS.
-//   * prefill_generic_kernel (everything else, incl. fp32): one lane per query
-//     row, fp32 FMA, K/V tiles staged through LDS.
-// Both compute, for query row i of (b, h) and keys j < Skv with
+//   * prefill_f32_kernel (fp32, D a multiple of 4 up to 128): the same on
+//     v_mfma_f32_32x32x2_f32, operands straight from L2.
+//   * prefill_generic_kernel (everything else): one lane per query row, fp32
+//     FMA, K/V tiles staged through LDS.
+// All compute, for query row i of (b, h) and keys j < Skv with
 // j <= i + q_offset: o = softmax(q.k_j * scale + bias_ij) v, lse = ln-sum-exp,
 // where the optional additive bias (an attention mask) is read through
 // broadcast strides.
@@ -14,6 +16,7 @@
 
 #include <type_traits>
 
+#include "attn_f32.h"
 #include "attn_tiles.h"
 #include "lc_common.h"
 
@@ -114,6 +117,154 @@ __global__ __launch_bounds__(64) void prefill_generic_kernel(PrefillArgs a) {
     if (d < a.D) op[d] = lc_from_f32<T>(acc[d] * inv);
   if (a.lse != nullptr)
     a.lse[((int64_t)b * a.Hq + h) * a.Sq + i] = l > 0.f ? (m + lc_log2(l)) * kLn2 : -INFINITY;
+}
+
+// ---------------------------------------------------------------------------
+// fp32 MFMA kernel (fp32, D a multiple of 4 up to 128).
+//
+// Workgroup = 4 waves on the same 32 query rows of one head; wave w takes the
+// 32-key tiles w, w + 4, .. and the four softmax states are merged through LDS
+// at the end, so a workgroup's waves finish together whatever its causal
+// length, no barrier stands in the loop, and short prompts still spread over
+// four SIMDs. Per tile and wave, all in fp32 (v_mfma_f32_32x32x2_f32; operand
+// forms in attn_f32.h): S^T = K Q^T, then the softmax (keys on accumulator
+// rows, queries on lanes), then O^T += V^T P^T.
+// Bound by the fp32 matrix rate (157 TF at 2.4 GHz; a softmax element costs
+// its SIMD about 1/20 of its MFMA time): V is loaded before the S products and
+// the next tile's K before the P V products, each covered by 2000 cycles of
+// MFMA at D = 64.
+// ---------------------------------------------------------------------------
+template <int DPAD, bool BIAS>
+__global__ __launch_bounds__(64 * kF32Waves) __attribute__((
+    amdgpu_waves_per_eu(DPAD <= 64 ? 2 : 1, DPAD <= 64 ? 2 : 1))) void
+prefill_f32_kernel(PrefillArgs a, int n_rb) {
+  constexpr int DTL = DPAD / 32, LD = DPAD + 4;
+  __shared__ __align__(16) float slab[kF32Waves][32 * LD];
+  __shared__ float ms[kF32Waves][32], ls[kF32Waves][32];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  // Heaviest row blocks first over all heads; a head's blocks share an XCD
+  // (block ids mod 8) where the heads are a multiple of 8.
+  const int units = gridDim.x / n_rb;
+  const int rank = blockIdx.x / units;
+  const int unit = blockIdx.x - rank * units;
+  const int b = unit / a.Hq, h = unit - b * a.Hq;
+  const int kvh = h / a.G;
+  const int r0 = (n_rb - 1 - rank) * kF32Rows;
+  const int qi = r0 + l32;
+  const bool row_ok = qi < a.Sq;
+  const int kv_end = min(a.Skv, min(a.Sq - 1, r0 + kF32Rows - 1) + a.q_offset + 1);
+  const int n_tiles = (kv_end + kF32Rows - 1) / kF32Rows;
+
+  const float* qb = static_cast<const float*>(a.q) + b * a.qs[0] + (int64_t)h * a.qs[1];
+  const float* kb = static_cast<const float*>(a.k) + b * a.ks[0] + (int64_t)kvh * a.ks[1];
+  const float* vb = static_cast<const float*>(a.v) + b * a.vs[0] + (int64_t)kvh * a.vs[1];
+  const __amdgpu_buffer_rsrc_t krs = f32_rsrc(kb, f32_bytes(a.Skv, a.ks[2], a.D));
+  const __amdgpu_buffer_rsrc_t vrs = f32_rsrc(vb, f32_bytes(a.Skv, a.vs[2], a.D));
+  const int ks_b = static_cast<int>(a.ks[2] * 4), vs_b = static_cast<int>(a.vs[2] * 4);
+  const int64_t brow = b * a.bs[0] + h * a.bs[1] + (int64_t)qi * a.bs[2];
+
+  F32Row<DPAD> q, k;
+  q.load(f32_rsrc(qb, f32_bytes(a.Sq, a.qs[2], a.D)), qi, static_cast<int>(a.qs[2] * 4), hh, a.D);
+  k.load(krs, wave * kF32Rows + l32, ks_b, hh, a.D);
+  f32x16_t o[DTL];
+#pragma unroll
+  for (int dt = 0; dt < DTL; ++dt) f32_zero(o[dt]);
+  float m = -INFINITY, l = 0.f;
+
+  for (int t = wave; t < n_tiles; t += kF32Waves) {
+    const int k0 = t * kF32Rows;
+    F32Cols<DTL> v;
+    v.load(vrs, k0, vs_b, l32, hh, a.D);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16_t s;
+    f32_zero(s);
+    f32_dot<DPAD>(s, k, q);
+    // (rows past the last key load as zeros)
+    k.load(krs, k0 + kF32Waves * kF32Rows + l32, ks_b, hh, a.D);
+    __builtin_amdgcn_sched_barrier(0);
+    // Scores in the exp2 domain; key k0 + c + 4hh is visible while c < key_lim.
+    const bool edge = k0 + kF32Rows - 1 > min(r0 + a.q_offset, a.Skv - 1);
+    const int key_lim = min(qi + a.q_offset + 1, a.Skv) - k0 - 4 * hh;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      s[r] *= a.scale_log2;
+      if constexpr (BIAS) {
+        const int c = 8 * (r >> 2) + (r & 3);
+        if (row_ok && c < key_lim)
+          s[r] += lc_bias_log2(
+              lc_load_bias(a.bias, brow + (int64_t)(k0 + c + 4 * hh) * a.bs[3], a.bias_dtype));
+      }
+    }
+    if (edge) {
+#pragma unroll
+      for (int r = 0; r < 16; ++r)
+        if (8 * (r >> 2) + (r & 3) >= key_lim) s[r] = -INFINITY;
+    }
+    float mx = -INFINITY;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+    const float m_new = fmaxf(m, pf_half_max(mx));
+    if (__ballot(m_new > m) != 0) {
+      const float alpha = m_new == -INFINITY ? 1.f : lc_exp2(m - m_new);
+      l *= alpha;
+#pragma unroll
+      for (int dt = 0; dt < DTL; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+      m = m_new;
+    }
+    const float m_use = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      float p = lc_exp2(s[r] - m_use);
+      if (BIAS || edge) p = s[r] == -INFINITY ? kF32Masked : p;
+      s[r] = p;
+      l += p;
+    }
+    if ((BIAS || edge) && v.any_nonfinite())
+      f32_outer_guarded<DTL>(o, vrs, k0, vs_b, s, slab[wave], l32, hh, a.D);
+    else
+      f32_outer<DTL>(o, v, s);
+  }
+
+  // Merge: o = sum_w 2^(m_w - M) O_w / sum_w 2^(m_w - M) l_w.
+  l += __shfl_xor(l, 32, 64);
+  f32_put<DPAD>(slab[wave], o, l32, hh);
+  if (hh == 0) {
+    ms[wave][l32] = m;
+    ls[wave][l32] = l;
+  }
+  __syncthreads();
+  constexpr int CPR = DPAD / 4;  // 4-dim chunks per row
+#pragma unroll
+  for (int e = tid; e < 32 * CPR; e += 64 * kF32Waves) {
+    const int row = e / CPR, d = (e - row * CPR) * 4;
+    if (r0 + row >= a.Sq || d >= a.D) continue;
+    float mt = -INFINITY, lt = 0.f;
+#pragma unroll
+    for (int w = 0; w < kF32Waves; ++w) mt = fmaxf(mt, ms[w][row]);
+    f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kF32Waves; ++w) {
+      // (a wave without a visible key holds zeros)
+      const float mw = ms[w][row];
+      const float f = mw == -INFINITY ? 0.f : lc_exp2(mw - mt);
+      lt = fmaf(ls[w][row], f, lt);
+      const f32x4_t ow = *reinterpret_cast<const f32x4_t*>(&slab[w][row * LD + d]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = fmaf(ow[i], f, acc[i]);
+    }
+    const float inv = lt > 0.f ? 1.0f / lt : 0.f;
+    float* orow = static_cast<float*>(a.o) + b * a.os[0] + (int64_t)h * a.os[1] +
+                  (int64_t)(r0 + row) * a.os[2];
+    *reinterpret_cast<f32x4_t*>(orow + d) = acc * inv;
+    if (d == 0 && a.lse != nullptr)
+      a.lse[((int64_t)b * a.Hq + h) * a.Sq + r0 + row] =
+          lt > 0.f ? (mt + lc_log2(lt)) * kLn2 : -INFINITY;
+  }
 }
 
 // ---------------------------------------------------------------------------
@@ -728,6 +879,27 @@ int launch_mfma(const PrefillArgs& a, hipStream_t st) {
   return lc_check_launch("lc_prefill_attn_fwd (mfma)");
 }
 
+template <int DPAD>
+void launch_f32_d(const PrefillArgs& a, unsigned nwg, int n_rb, hipStream_t st) {
+  if (a.bias == nullptr)
+    prefill_f32_kernel<DPAD, false><<<nwg, 64 * kF32Waves, 0, st>>>(a, n_rb);
+  else
+    prefill_f32_kernel<DPAD, true><<<nwg, 64 * kF32Waves, 0, st>>>(a, n_rb);
+}
+
+int launch_f32(const PrefillArgs& a, hipStream_t st) {
+  const int n_rb = (a.Sq + kF32Rows - 1) / kF32Rows;
+  const int64_t nwg = (int64_t)n_rb * a.Hq * a.B;
+  LC_REQUIRE(nwg < (1LL << 31), "lc_prefill_attn_fwd: grid too large");
+  if (a.D <= 32)
+    launch_f32_d<32>(a, (unsigned)nwg, n_rb, st);
+  else if (a.D <= 64)
+    launch_f32_d<64>(a, (unsigned)nwg, n_rb, st);
+  else
+    launch_f32_d<128>(a, (unsigned)nwg, n_rb, st);
+  return lc_check_launch("lc_prefill_attn_fwd (f32)");
+}
+
 template <typename T>
 int launch_generic(const PrefillArgs& a, hipStream_t st) {
   dim3 grid((a.Sq + 63) / 64, a.Hq, a.B);
@@ -829,9 +1001,20 @@ int lc_prefill_attn_fwd(const void* q, const void* k, const void* v, void* o, fl
     a.bias_vec = s3 == 1 && Skv % 4 == 0 && s2 % 4 == 0 && a.bs[0] % 4 == 0 &&
                  a.bs[1] % 4 == 0 && lc_aligned(bias, 4 * besz);
   }
+  // fp32 MFMA path: D a multiple of 4 up to 128, one head's q, k and v rows
+  // (the tiles past the last one that are loaded as zeros included) within
+  // 32-bit byte offsets, 16-byte aligned output rows. Both sides measured at
+  // [2, 16/8, 1024, 64]: 62 us against 987 us for the lane-per-row kernel,
+  // which keeps the other head_dims.
+  bool f32 = D % 4 == 0 && D <= 128 && lc_aligned(o, 16);
+  for (int i = 0; i < 3; ++i) f32 = f32 && o_strides[i] % 4 == 0;
+  const int64_t past = 2 * kF32Waves * kF32Rows;
+  f32 = f32 && ((Skv + past) * k_strides[2] + D) * 4 < kF32Oob &&
+        ((Skv + past) * v_strides[2] + D) * 4 < kF32Oob &&
+        ((Sq + past) * q_strides[2] + D) * 4 < kF32Oob;
   switch (dtype) {
     case LC_DTYPE_F32:
-      return launch_generic<float>(a, st);
+      return f32 ? launch_f32(a, st) : launch_generic<float>(a, st);
     case LC_DTYPE_BF16:
       return mfma ? launch_mfma<bf16_t>(a, st) : launch_generic<bf16_t>(a, st);
     case LC_DTYPE_F16:

@@ -19,11 +19,14 @@
 //     (Q/dO tiles in LDS, K^T and V^T operands in registers, queries on
 //     accumulator rows, keys on lanes), so in both the probabilities and dS
 //     feed the next product straight from the accumulator registers.
+//   * fp32 with D a multiple of 4 up to 128: the same two kernels on
+//     v_mfma_f32_32x32x2_f32, operands straight from L2 (attn_f32.h).
 //   * everything else: lane-per-row fp32 kernels.
 #include <math.h>
 
 #include <type_traits>
 
+#include "attn_f32.h"
 #include "attn_tiles.h"
 #include "lc_common.h"
 
@@ -301,6 +304,264 @@ int launch_bwd_generic(const BwdArgs& a, hipStream_t st) {
     LC_BWD_GEN(256);
 #undef LC_BWD_GEN
   return lc_check_launch("lc_prefill_attn_bwd (generic)");
+}
+
+// ---------------------------------------------------------------------------
+// fp32 MFMA kernels (fp32, D a multiple of 4 up to 128; operand forms in
+// attn_f32.h). A workgroup's 4 waves share one 32-row block and take every
+// fourth tile each; their sums are added through LDS at the end. Bound by the
+// fp32 matrix rate: 3 products per tile in the dQ kernel, 4 in the dK/dV one.
+// ---------------------------------------------------------------------------
+
+// The 4 waves' accumulators (dims x 32 columns), added in wave order and
+// scaled, to rows row0 .. of `out`. Ends with the slab free again.
+template <int DPAD>
+__device__ __forceinline__ void f32_store_sum(float* slab, int wave, int tid,
+                                              const f32x16_t (&acc)[DPAD / 32], float* out,
+                                              int64_t stride, int row0, int rows, int D,
+                                              float mul) {
+  constexpr int LD = DPAD + 4, CPR = DPAD / 4;
+  f32_put<DPAD>(slab + wave * 32 * LD, acc, tid & 31, (tid & 63) >> 5);
+  __syncthreads();
+#pragma unroll
+  for (int e = tid; e < 32 * CPR; e += 64 * kF32Waves) {
+    const int row = e / CPR, d = (e - row * CPR) * 4;
+    if (row0 + row >= rows || d >= D) continue;
+    f32x4_t sum = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int w = 0; w < kF32Waves; ++w)
+      sum += *reinterpret_cast<const f32x4_t*>(slab + w * 32 * LD + row * LD + d);
+    *reinterpret_cast<f32x4_t*>(out + (int64_t)(row0 + row) * stride + d) = sum * mul;
+  }
+  __syncthreads();
+}
+
+template <int DPAD, bool BIAS>
+__global__ __launch_bounds__(64 * kF32Waves) __attribute__((
+    amdgpu_waves_per_eu(DPAD <= 64 ? 2 : 1, DPAD <= 64 ? 2 : 1))) void
+attn_bwd_dq_f32_kernel(BwdArgs a, int n_rb) {
+  constexpr int DTL = DPAD / 32;
+  __shared__ __align__(16) float slab[kF32Waves * 32 * (DPAD + 4)];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  // Heaviest row blocks first over all heads, as in the forward.
+  const int units = gridDim.x / n_rb;
+  const int rank = blockIdx.x / units;
+  const int unit = blockIdx.x - rank * units;
+  const int b = unit / a.Hq, h = unit - b * a.Hq;
+  const int kvh = h / a.G;
+  const int r0 = (n_rb - 1 - rank) * kF32Rows;
+  const int qi = r0 + l32;
+  const bool row_ok = qi < a.Sq;
+  const int kv_end = min(a.Skv, min(a.Sq - 1, r0 + kF32Rows - 1) + a.q_offset + 1);
+  const int n_tiles = (kv_end + kF32Rows - 1) / kF32Rows;
+
+  const float* qb = static_cast<const float*>(a.q) + b * a.qs[0] + (int64_t)h * a.qs[1];
+  const float* ob = static_cast<const float*>(a.dout) + b * a.dos[0] + (int64_t)h * a.dos[1];
+  const float* kb = static_cast<const float*>(a.k) + b * a.ks[0] + (int64_t)kvh * a.ks[1];
+  const float* vb = static_cast<const float*>(a.v) + b * a.vs[0] + (int64_t)kvh * a.vs[1];
+  const __amdgpu_buffer_rsrc_t krs = f32_rsrc(kb, f32_bytes(a.Skv, a.ks[2], a.D));
+  const __amdgpu_buffer_rsrc_t vrs = f32_rsrc(vb, f32_bytes(a.Skv, a.vs[2], a.D));
+  const int ks_b = static_cast<int>(a.ks[2] * 4), vs_b = static_cast<int>(a.vs[2] * 4);
+  const int64_t brow = b * a.bs[0] + h * a.bs[1] + (int64_t)qi * a.bs[2];
+  const int64_t ridx = ((int64_t)b * a.Hq + h) * a.Sq + qi;
+  // (+inf for rows past the end and rows that saw no key: they get no gradient)
+  const float lse2 = row_ok ? a.lse2[ridx] : INFINITY;
+  const float dl = row_ok ? a.delta[ridx] : 0.f;
+
+  F32Row<DPAD> q, dout, k, v;
+  q.load(f32_rsrc(qb, f32_bytes(a.Sq, a.qs[2], a.D)), qi, static_cast<int>(a.qs[2] * 4), hh, a.D);
+  dout.load(f32_rsrc(ob, f32_bytes(a.Sq, a.dos[2], a.D)), qi, static_cast<int>(a.dos[2] * 4), hh,
+            a.D);
+  v.load(vrs, wave * kF32Rows + l32, vs_b, hh, a.D);
+  f32x16_t dq[DTL];
+#pragma unroll
+  for (int dt = 0; dt < DTL; ++dt) f32_zero(dq[dt]);
+
+  for (int t = wave; t < n_tiles; t += kF32Waves) {
+    const int k0 = t * kF32Rows;
+    k.load(krs, k0 + l32, ks_b, hh, a.D);
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16_t s, dp;
+    f32_zero(dp);
+    f32_dot<DPAD>(dp, v, dout);  // covers the K rows' latency
+    F32Cols<DTL> kc;
+    kc.load(krs, k0, ks_b, l32, hh, a.D);
+    v.load(vrs, k0 + kF32Waves * kF32Rows + l32, vs_b, hh, a.D);
+    __builtin_amdgcn_sched_barrier(0);
+    f32_zero(s);
+    f32_dot<DPAD>(s, k, q);
+    const bool edge = k0 + kF32Rows - 1 > min(r0 + a.q_offset, a.Skv - 1);
+    const int key_lim = min(qi + a.q_offset + 1, a.Skv) - k0 - 4 * hh;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      const int c = 8 * (r >> 2) + (r & 3);
+      float x = s[r] * a.scale_log2 - lse2;
+      bool masked = lse2 == INFINITY;
+      if constexpr (BIAS) {
+        if (row_ok && c < key_lim) {
+          const float bias = lc_bias_log2(
+              lc_load_bias(a.bias, brow + (int64_t)(k0 + c + 4 * hh) * a.bs[3], a.bias_dtype));
+          x += bias;
+          masked = masked || bias == -INFINITY;
+        }
+      }
+      if (edge) masked = masked || c >= key_lim;
+      const float ds = lc_exp2(x) * (dp[r] - dl);
+      s[r] = masked ? kF32Masked : ds;
+    }
+    if ((BIAS || edge) && kc.any_nonfinite())
+      f32_outer_guarded<DTL>(dq, krs, k0, ks_b, s, slab + wave * 32 * (DPAD + 4), l32, hh, a.D);
+    else
+      f32_outer<DTL>(dq, kc, s);
+  }
+  f32_store_sum<DPAD>(slab, wave, tid, dq,
+                      static_cast<float*>(a.dq) + b * a.dqs[0] + (int64_t)h * a.dqs[1], a.dqs[2],
+                      r0, a.Sq, a.D, a.scale);
+}
+
+// The waves' tiles are the (query tile, head of the group) pairs that see the
+// 32-key block, dealt round robin.
+template <int DPAD, bool BIAS>
+__global__ __launch_bounds__(64 * kF32Waves) __attribute__((
+    amdgpu_waves_per_eu(DPAD <= 32 ? 2 : 1, DPAD <= 32 ? 2 : 1))) void
+attn_bwd_dkv_f32_kernel(BwdArgs a, int n_kb, int cus) {
+  constexpr int DTL = DPAD / 32;
+  __shared__ __align__(16) float slab[kF32Waves * 32 * (DPAD + 4)];
+  __shared__ __align__(16) float rows_lds[kF32Waves][64];
+  const int tid = threadIdx.x;
+  const int lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int l32 = lane & 31, hh = lane >> 5;
+  // Heaviest (earliest) key blocks first over all kv heads.
+  const int units = gridDim.x / n_kb;
+  const int lin = f32_snake(blockIdx.x, gridDim.x, cus);
+  const int kblk = lin / units;
+  const int unit = lin - kblk * units;
+  const int b = unit / a.Hkv, kvh = unit - b * a.Hkv;
+  const int key0 = kblk * kF32Rows;
+  const int kj = key0 + l32;
+
+  const float* kb = static_cast<const float*>(a.k) + b * a.ks[0] + (int64_t)kvh * a.ks[1];
+  const float* vb = static_cast<const float*>(a.v) + b * a.vs[0] + (int64_t)kvh * a.vs[1];
+  const int qs_b = static_cast<int>(a.qs[2] * 4), os_b = static_cast<int>(a.dos[2] * 4);
+  const int q_bytes = f32_bytes(a.Sq, a.qs[2], a.D), o_bytes = f32_bytes(a.Sq, a.dos[2], a.D);
+  F32Row<DPAD> k, v;
+  k.load(f32_rsrc(kb, f32_bytes(a.Skv, a.ks[2], a.D)), kj, static_cast<int>(a.ks[2] * 4), hh, a.D);
+  v.load(f32_rsrc(vb, f32_bytes(a.Skv, a.vs[2], a.D)), kj, static_cast<int>(a.vs[2] * 4), hh, a.D);
+  f32x16_t dk[DTL], dv[DTL];
+#pragma unroll
+  for (int dt = 0; dt < DTL; ++dt) {
+    f32_zero(dk[dt]);
+    f32_zero(dv[dt]);
+  }
+  const int qt0 = max(0, key0 - a.q_offset) / kF32Rows;
+  const int n_qt = (a.Sq + kF32Rows - 1) / kF32Rows;
+  const int n_iter = max(0, n_qt - qt0) * a.G;
+
+  for (int it = wave; it < n_iter; it += kF32Waves) {
+    const int step = it / a.G;
+    const int q0 = (n_qt - 1 - step) * kF32Rows;
+    const int h = kvh * a.G + (it - step * a.G);
+    const __amdgpu_buffer_rsrc_t qrs = f32_rsrc(
+        static_cast<const float*>(a.q) + b * a.qs[0] + (int64_t)h * a.qs[1], q_bytes);
+    const __amdgpu_buffer_rsrc_t ors = f32_rsrc(
+        static_cast<const float*>(a.dout) + b * a.dos[0] + (int64_t)h * a.dos[1], o_bytes);
+    F32Row<DPAD> qr, dor;
+    qr.load(qrs, q0 + l32, qs_b, hh, a.D);
+    dor.load(ors, q0 + l32, os_b, hh, a.D);
+    // lse2 of the tile's rows in lanes 0-31, delta in lanes 32-63 (rows past
+    // the end: probability 0).
+    const int qi = q0 + l32;
+    const float* rsrc = (hh == 0 ? a.lse2 : a.delta) + ((int64_t)b * a.Hq + h) * a.Sq;
+    const float rv = qi < a.Sq ? rsrc[qi] : (hh == 0 ? INFINITY : 0.f);
+    F32Cols<DTL> oc, qc;
+    auto load_cols = [&]() __attribute__((always_inline)) {
+      oc.load(ors, q0, os_b, l32, hh, a.D);
+      qc.load(qrs, q0, qs_b, l32, hh, a.D);
+    };
+    // (at D 128 both forms of the tile do not fit the registers at once)
+    if constexpr (DPAD <= 64) load_cols();
+    __builtin_amdgcn_sched_barrier(0);
+    f32x16_t s, dp;
+    f32_zero(s);
+    f32_zero(dp);
+    f32_dot<DPAD>(s, qr, k);
+    rows_lds[wave][lane] = rv;
+    f32_dot<DPAD>(dp, dor, v);
+    if constexpr (DPAD > 64) load_cols();
+    lc_compiler_fence();
+    const bool edge = q0 + a.q_offset < key0 + kF32Rows - 1;
+    const int row_lim = kj - q0 - a.q_offset - 4 * hh;  // row c + 4hh sees the key from c = row_lim on
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&rows_lds[wave][8 * j + 4 * hh]);
+      const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&rows_lds[wave][32 + 8 * j + 4 * hh]);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int r = 4 * j + i, c = 8 * j + i;
+        float x = s[r] * a.scale_log2 - l4[i];
+        bool masked = edge && c < row_lim;
+        if constexpr (BIAS) {
+          const int row = q0 + c + 4 * hh;
+          if (!masked && row < a.Sq && kj < a.Skv) {
+            const float bias = lc_bias_log2(lc_load_bias(
+                a.bias, b * a.bs[0] + h * a.bs[1] + (int64_t)row * a.bs[2] + (int64_t)kj * a.bs[3],
+                a.bias_dtype));
+            x += bias;
+            masked = bias == -INFINITY;
+          }
+        }
+        const float p = lc_exp2(x);
+        s[r] = masked ? kF32Masked : p;
+        dp[r] = masked ? kF32Masked : p * (dp[r] - d4[i]);
+      }
+    }
+    lc_compiler_fence();
+    float* scratch = slab + wave * 32 * (DPAD + 4);
+    if ((BIAS || edge) && (oc.any_nonfinite() || qc.any_nonfinite())) {
+      f32_outer_guarded<DTL>(dv, ors, q0, os_b, s, scratch, l32, hh, a.D);
+      f32_outer_guarded<DTL>(dk, qrs, q0, qs_b, dp, scratch, l32, hh, a.D);
+    } else {
+      f32_outer<DTL>(dv, oc, s);
+      f32_outer<DTL>(dk, qc, dp);
+    }
+  }
+  f32_store_sum<DPAD>(slab, wave, tid, dk,
+                      static_cast<float*>(a.dk) + b * a.dks[0] + (int64_t)kvh * a.dks[1], a.dks[2],
+                      key0, a.Skv, a.D, a.scale);
+  f32_store_sum<DPAD>(slab, wave, tid, dv,
+                      static_cast<float*>(a.dv) + b * a.dvs[0] + (int64_t)kvh * a.dvs[1], a.dvs[2],
+                      key0, a.Skv, a.D, 1.0f);
+}
+
+template <int DPAD, bool BIAS>
+void launch_bwd_f32_d(const BwdArgs& a, hipStream_t st) {
+  const int n_rb = (a.Sq + kF32Rows - 1) / kF32Rows, n_kb = (a.Skv + kF32Rows - 1) / kF32Rows;
+  if (n_rb > 0)
+    attn_bwd_dq_f32_kernel<DPAD, BIAS>
+        <<<(unsigned)(n_rb * a.Hq * a.B), 64 * kF32Waves, 0, st>>>(a, n_rb);
+  if (n_kb > 0)
+    attn_bwd_dkv_f32_kernel<DPAD, BIAS>
+        <<<(unsigned)(n_kb * a.Hkv * a.B), 64 * kF32Waves, 0, st>>>(a, n_kb, lc_cu_count());
+}
+
+int launch_bwd_f32(const BwdArgs& a, hipStream_t st) {
+  const int64_t n_rb = (a.Sq + kF32Rows - 1) / kF32Rows, n_kb = (a.Skv + kF32Rows - 1) / kF32Rows;
+  LC_REQUIRE(n_rb * a.Hq * a.B < (1LL << 31) && n_kb * a.Hkv * a.B < (1LL << 31),
+             "lc_prefill_attn_bwd: grid too large");
+#define LC_BWD_F32(DP) \
+  (a.bias == nullptr ? launch_bwd_f32_d<DP, false>(a, st) : launch_bwd_f32_d<DP, true>(a, st))
+  if (a.D <= 32)
+    LC_BWD_F32(32);
+  else if (a.D <= 64)
+    LC_BWD_F32(64);
+  else
+    LC_BWD_F32(128);
+#undef LC_BWD_F32
+  return lc_check_launch("lc_prefill_attn_bwd (f32)");
 }
 
 // ---------------------------------------------------------------------------
@@ -1100,6 +1361,9 @@ int run_bwd(const void* o, const int64_t* o_strides, BwdArgs a, float* delta, fl
   }
   int rc = launch_delta<T>(o, o_strides, a, delta, lse2, st);
   if (rc != LC_OK) return rc;
+  if constexpr (std::is_same<T, float>::value) {
+    if (mfma) return launch_bwd_f32(a, st);
+  }
   return launch_bwd_generic<T>(a, st);
 }
 
@@ -1211,10 +1475,23 @@ int lc_prefill_attn_bwd(const void* q, const void* k, const void* v, const void*
     a.bias_vec = s3 == 1 && Skv % 4 == 0 && s2 % 4 == 0 && a.bs[0] % 4 == 0 &&
                  a.bs[1] % 4 == 0 && lc_aligned(bias, 4 * besz);
   }
+  // fp32 MFMA kernels: D a multiple of 4 up to 128, 16-byte aligned output
+  // rows, one head's rows (and the zero tiles past them) within 32-bit byte
+  // offsets. At [2, 16/8, 1024, 64] 267 us against 3193 us for the lane-per-row
+  // kernels, which keep the other head_dims.
+  bool f32 = D % 4 == 0 && D <= 128 && lc_aligned(dq, 16) && lc_aligned(dk, 16) &&
+             lc_aligned(dv, 16);
+  const int64_t past = 2 * kF32Waves * kF32Rows;
+  for (int i = 0; i < 3; ++i)
+    f32 = f32 && dq_strides[i] % 4 == 0 && dk_strides[i] % 4 == 0 && dv_strides[i] % 4 == 0;
+  for (const int64_t rs : {k_strides[2], v_strides[2]})
+    f32 = f32 && ((Skv + past) * rs + D) * 4 < kF32Oob;
+  for (const int64_t rs : {q_strides[2], do_strides[2]})
+    f32 = f32 && ((Sq + past) * rs + D) * 4 < kF32Oob;
   hipStream_t st = lc_stream(stream);
   switch (dtype) {
     case LC_DTYPE_F32:
-      return run_bwd<float>(o, o_strides, a, delta, lse2, false, st);
+      return run_bwd<float>(o, o_strides, a, delta, lse2, f32, st);
     case LC_DTYPE_BF16:
       return run_bwd<bf16_t>(o, o_strides, a, delta, lse2, mfma, st);
     case LC_DTYPE_F16:
