@@ -75,6 +75,33 @@ __device__ __forceinline__ void f32_dot(f32x16_t& acc, const F32Row<DPAD>& A,
     for (int e = 0; e < 4; ++e) acc = f32_mma(A.c[i][e], B.c[i][e], acc);
 }
 
+// 32 rows from row0 on into LDS, DPAD + 4 floats apart (the whole workgroup;
+// rows past the range and dims past D: zeros).
+template <int DPAD>
+__device__ __forceinline__ void f32_stage(float* dst, const float* base, int nbytes, int row0,
+                                          int stride_b, int tid, int D) {
+  const __amdgpu_buffer_rsrc_t rs = f32_rsrc(base, nbytes);
+#pragma unroll
+  for (int e = tid; e < 32 * (DPAD / 4); e += 64 * kF32Waves) {
+    const int row = e / (DPAD / 4), d = (e - row * (DPAD / 4)) * 4;
+    const int off = d < D ? (row0 + row) * stride_b + d * 4 : kF32Oob;
+    *reinterpret_cast<u32x4_t*>(dst + row * (DPAD + 4) + d) =
+        __builtin_amdgcn_raw_buffer_load_b128(rs, off, 0, 0);
+  }
+}
+
+// f32_dot with B rows staged by f32_stage (b: the lane's row + 4 hh).
+template <int DPAD>
+__device__ __forceinline__ void f32_dot_lds(f32x16_t& acc, const F32Row<DPAD>& A,
+                                            const float* b) {
+#pragma unroll
+  for (int i = 0; i < DPAD / 8; ++i) {
+    const f32x4_t B = *reinterpret_cast<const f32x4_t*>(b + i * 8);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) acc = f32_mma(A.c[i][e], B[e], acc);
+  }
+}
+
 template <int DTL>
 struct F32Dims {
   float v[DTL];
@@ -95,11 +122,13 @@ struct F32Cols {
   F32Dims<DTL> n[16];
   __device__ __forceinline__ void load(__amdgpu_buffer_rsrc_t rs, int row0, int stride_b, int l32,
                                        int hh, int D) {
-    const int base = (row0 + 4 * hh) * stride_b + l32 * DTL * 4;
+    // (dims past D: out of range from any row of the tile, without a wrap)
+    const int base = l32 * DTL < D ? (row0 + 4 * hh) * stride_b + l32 * DTL * 4 : kF32Oob;
 #pragma unroll
     for (int r = 0; r < 16; ++r)
       n[r] = f32_load_dims<DTL>(
-          rs, l32 * DTL < D ? base + (8 * (r >> 2) + (r & 3)) * stride_b : kF32Oob);
+          rs, static_cast<int>(static_cast<unsigned>(base) +
+                               static_cast<unsigned>((8 * (r >> 2) + (r & 3)) * stride_b)));
   }
   // Whether any value of the tile is infinite or NaN (in any lane).
   __device__ __forceinline__ bool any_nonfinite() const {

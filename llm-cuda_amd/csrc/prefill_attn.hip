@@ -188,42 +188,46 @@ prefill_f32_kernel(PrefillArgs a, int n_rb) {
     // Scores in the exp2 domain; key k0 + c + 4hh is visible while c < key_lim.
     const bool edge = k0 + kF32Rows - 1 > min(r0 + a.q_offset, a.Skv - 1);
     const int key_lim = min(qi + a.q_offset + 1, a.Skv) - k0 - 4 * hh;
+    // MASK: some pair may be masked (the diagonal, the last keys, a bias).
+    auto softmax = [&](auto mask_c) __attribute__((always_inline)) {
+      constexpr bool MASK = decltype(mask_c)::value;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      s[r] *= a.scale_log2;
-      if constexpr (BIAS) {
+      for (int r = 0; r < 16; ++r) {
         const int c = 8 * (r >> 2) + (r & 3);
-        if (row_ok && c < key_lim)
-          s[r] += lc_bias_log2(
-              lc_load_bias(a.bias, brow + (int64_t)(k0 + c + 4 * hh) * a.bs[3], a.bias_dtype));
+        s[r] *= a.scale_log2;
+        if constexpr (BIAS) {
+          if (row_ok && c < key_lim)
+            s[r] += lc_bias_log2(
+                lc_load_bias(a.bias, brow + (int64_t)(k0 + c + 4 * hh) * a.bs[3], a.bias_dtype));
+        }
+        if (MASK && c >= key_lim) s[r] = -INFINITY;
       }
-    }
-    if (edge) {
+      float mx = -INFINITY;
 #pragma unroll
-      for (int r = 0; r < 16; ++r)
-        if (8 * (r >> 2) + (r & 3) >= key_lim) s[r] = -INFINITY;
-    }
-    float mx = -INFINITY;
+      for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
+      const float m_new = fmaxf(m, pf_half_max(mx));
+      if (__ballot(m_new > m) != 0) {
+        const float alpha = m_new == -INFINITY ? 1.f : lc_exp2(m - m_new);
+        l *= alpha;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) mx = fmaxf(mx, s[r]);
-    const float m_new = fmaxf(m, pf_half_max(mx));
-    if (__ballot(m_new > m) != 0) {
-      const float alpha = m_new == -INFINITY ? 1.f : lc_exp2(m - m_new);
-      l *= alpha;
+        for (int dt = 0; dt < DTL; ++dt)
 #pragma unroll
-      for (int dt = 0; dt < DTL; ++dt)
+          for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
+        m = m_new;
+      }
+      const float m_use = m == -INFINITY ? 0.f : m;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) o[dt][r] *= alpha;
-      m = m_new;
-    }
-    const float m_use = m == -INFINITY ? 0.f : m;
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      float p = lc_exp2(s[r] - m_use);
-      if (BIAS || edge) p = s[r] == -INFINITY ? kF32Masked : p;
-      s[r] = p;
-      l += p;
-    }
+      for (int r = 0; r < 16; ++r) {
+        float p = lc_exp2(s[r] - m_use);
+        if (MASK) p = s[r] == -INFINITY ? kF32Masked : p;
+        s[r] = p;
+        l += p;
+      }
+    };
+    if (BIAS || edge)
+      softmax(std::true_type{});
+    else
+      softmax(std::false_type{});
     if ((BIAS || edge) && v.any_nonfinite())
       f32_outer_guarded<DTL>(o, vrs, k0, vs_b, s, slab[wave], l32, hh, a.D);
     else
@@ -1004,7 +1008,7 @@ int lc_prefill_attn_fwd(const void* q, const void* k, const void* v, void* o, fl
   // fp32 MFMA path: D a multiple of 4 up to 128, one head's q, k and v rows
   // (the tiles past the last one that are loaded as zeros included) within
   // 32-bit byte offsets, 16-byte aligned output rows. Both sides measured at
-  // [2, 16/8, 1024, 64]: 62 us against 987 us for the lane-per-row kernel,
+  // [2, 16/8, 1024, 64]: 55 us against 987 us for the lane-per-row kernel,
   // which keeps the other head_dims.
   bool f32 = D % 4 == 0 && D <= 128 && lc_aligned(o, 16);
   for (int i = 0; i < 3; ++i) f32 = f32 && o_strides[i] % 4 == 0;

@@ -370,6 +370,7 @@ attn_bwd_dq_f32_kernel(BwdArgs a, int n_rb) {
   // (+inf for rows past the end and rows that saw no key: they get no gradient)
   const float lse2 = row_ok ? a.lse2[ridx] : INFINITY;
   const float dl = row_ok ? a.delta[ridx] : 0.f;
+  const bool no_key = lse2 == INFINITY;
 
   F32Row<DPAD> q, dout, k, v;
   q.load(f32_rsrc(qb, f32_bytes(a.Sq, a.qs[2], a.D)), qi, static_cast<int>(a.qs[2] * 4), hh, a.D);
@@ -395,23 +396,29 @@ attn_bwd_dq_f32_kernel(BwdArgs a, int n_rb) {
     f32_dot<DPAD>(s, k, q);
     const bool edge = k0 + kF32Rows - 1 > min(r0 + a.q_offset, a.Skv - 1);
     const int key_lim = min(qi + a.q_offset + 1, a.Skv) - k0 - 4 * hh;
+    auto softmax_grad = [&](auto mask_c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int c = 8 * (r >> 2) + (r & 3);
-      float x = s[r] * a.scale_log2 - lse2;
-      bool masked = lse2 == INFINITY;
-      if constexpr (BIAS) {
-        if (row_ok && c < key_lim) {
-          const float bias = lc_bias_log2(
-              lc_load_bias(a.bias, brow + (int64_t)(k0 + c + 4 * hh) * a.bs[3], a.bias_dtype));
-          x += bias;
-          masked = masked || bias == -INFINITY;
+      for (int r = 0; r < 16; ++r) {
+        const int c = 8 * (r >> 2) + (r & 3);
+        float x = s[r] * a.scale_log2 - lse2;
+        bool masked = no_key;
+        if constexpr (BIAS) {
+          if (row_ok && c < key_lim) {
+            const float bias = lc_bias_log2(
+                lc_load_bias(a.bias, brow + (int64_t)(k0 + c + 4 * hh) * a.bs[3], a.bias_dtype));
+            x += bias;
+            masked = masked || bias == -INFINITY;
+          }
         }
+        if (decltype(mask_c)::value) masked = masked || c >= key_lim;
+        const float ds = lc_exp2(x) * (dp[r] - dl);
+        s[r] = masked ? kF32Masked : ds;
       }
-      if (edge) masked = masked || c >= key_lim;
-      const float ds = lc_exp2(x) * (dp[r] - dl);
-      s[r] = masked ? kF32Masked : ds;
-    }
+    };
+    if (BIAS || edge)
+      softmax_grad(std::true_type{});
+    else
+      softmax_grad(std::false_type{});
     if ((BIAS || edge) && kc.any_nonfinite())
       f32_outer_guarded<DTL>(dq, krs, k0, ks_b, s, slab + wave * 32 * (DPAD + 4), l32, hh, a.D);
     else
@@ -426,11 +433,12 @@ attn_bwd_dq_f32_kernel(BwdArgs a, int n_rb) {
 // 32-key block, dealt round robin.
 template <int DPAD, bool BIAS>
 __global__ __launch_bounds__(64 * kF32Waves) __attribute__((
-    amdgpu_waves_per_eu(DPAD <= 32 ? 2 : 1, DPAD <= 32 ? 2 : 1))) void
+    amdgpu_waves_per_eu(DPAD <= 64 ? 2 : 1, DPAD <= 64 ? 2 : 1))) void
 attn_bwd_dkv_f32_kernel(BwdArgs a, int n_kb, int cus) {
-  constexpr int DTL = DPAD / 32;
+  constexpr int DTL = DPAD / 32, LD = DPAD + 4;
   __shared__ __align__(16) float slab[kF32Waves * 32 * (DPAD + 4)];
   __shared__ __align__(16) float rows_lds[kF32Waves][64];
+  __shared__ __align__(16) float k_lds[32 * LD], v_lds[32 * LD];
   const int tid = threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -448,9 +456,13 @@ attn_bwd_dkv_f32_kernel(BwdArgs a, int n_kb, int cus) {
   const float* vb = static_cast<const float*>(a.v) + b * a.vs[0] + (int64_t)kvh * a.vs[1];
   const int qs_b = static_cast<int>(a.qs[2] * 4), os_b = static_cast<int>(a.dos[2] * 4);
   const int q_bytes = f32_bytes(a.Sq, a.qs[2], a.D), o_bytes = f32_bytes(a.Sq, a.dos[2], a.D);
-  F32Row<DPAD> k, v;
-  k.load(f32_rsrc(kb, f32_bytes(a.Skv, a.ks[2], a.D)), kj, static_cast<int>(a.ks[2] * 4), hh, a.D);
-  v.load(f32_rsrc(vb, f32_bytes(a.Skv, a.vs[2], a.D)), kj, static_cast<int>(a.vs[2] * 4), hh, a.D);
+  // The block's K and V rows, the B operands of every tile, stay in LDS (64
+  // registers a wave that two waves per SIMD do not have).
+  f32_stage<DPAD>(k_lds, kb, f32_bytes(a.Skv, a.ks[2], a.D), key0, static_cast<int>(a.ks[2] * 4),
+                  tid, a.D);
+  f32_stage<DPAD>(v_lds, vb, f32_bytes(a.Skv, a.vs[2], a.D), key0, static_cast<int>(a.vs[2] * 4),
+                  tid, a.D);
+  __syncthreads();
   f32x16_t dk[DTL], dv[DTL];
 #pragma unroll
   for (int dt = 0; dt < DTL; ++dt) {
@@ -478,47 +490,49 @@ attn_bwd_dkv_f32_kernel(BwdArgs a, int n_kb, int cus) {
     const float* rsrc = (hh == 0 ? a.lse2 : a.delta) + ((int64_t)b * a.Hq + h) * a.Sq;
     const float rv = qi < a.Sq ? rsrc[qi] : (hh == 0 ? INFINITY : 0.f);
     F32Cols<DTL> oc, qc;
-    auto load_cols = [&]() __attribute__((always_inline)) {
-      oc.load(ors, q0, os_b, l32, hh, a.D);
-      qc.load(qrs, q0, qs_b, l32, hh, a.D);
-    };
-    // (at D 128 both forms of the tile do not fit the registers at once)
-    if constexpr (DPAD <= 64) load_cols();
+    oc.load(ors, q0, os_b, l32, hh, a.D);
     __builtin_amdgcn_sched_barrier(0);
     f32x16_t s, dp;
     f32_zero(s);
     f32_zero(dp);
-    f32_dot<DPAD>(s, qr, k);
+    f32_dot_lds<DPAD>(s, qr, k_lds + l32 * LD + hh * 4);
     rows_lds[wave][lane] = rv;
-    f32_dot<DPAD>(dp, dor, v);
-    if constexpr (DPAD > 64) load_cols();
+    qc.load(qrs, q0, qs_b, l32, hh, a.D);  // (into the registers of qr)
+    __builtin_amdgcn_sched_barrier(0);
+    f32_dot_lds<DPAD>(dp, dor, v_lds + l32 * LD + hh * 4);
     lc_compiler_fence();
     const bool edge = q0 + a.q_offset < key0 + kF32Rows - 1;
     const int row_lim = kj - q0 - a.q_offset - 4 * hh;  // row c + 4hh sees the key from c = row_lim on
+    auto softmax_grad = [&](auto mask_c) __attribute__((always_inline)) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&rows_lds[wave][8 * j + 4 * hh]);
-      const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&rows_lds[wave][32 + 8 * j + 4 * hh]);
+      for (int j = 0; j < 4; ++j) {
+        const f32x4_t l4 = *reinterpret_cast<const f32x4_t*>(&rows_lds[wave][8 * j + 4 * hh]);
+        const f32x4_t d4 = *reinterpret_cast<const f32x4_t*>(&rows_lds[wave][32 + 8 * j + 4 * hh]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int r = 4 * j + i, c = 8 * j + i;
-        float x = s[r] * a.scale_log2 - l4[i];
-        bool masked = edge && c < row_lim;
-        if constexpr (BIAS) {
-          const int row = q0 + c + 4 * hh;
-          if (!masked && row < a.Sq && kj < a.Skv) {
-            const float bias = lc_bias_log2(lc_load_bias(
-                a.bias, b * a.bs[0] + h * a.bs[1] + (int64_t)row * a.bs[2] + (int64_t)kj * a.bs[3],
-                a.bias_dtype));
-            x += bias;
-            masked = bias == -INFINITY;
+        for (int i = 0; i < 4; ++i) {
+          const int r = 4 * j + i, c = 8 * j + i;
+          float x = s[r] * a.scale_log2 - l4[i];
+          bool masked = decltype(mask_c)::value && c < row_lim;
+          if constexpr (BIAS) {
+            const int row = q0 + c + 4 * hh;
+            if (!masked && row < a.Sq && kj < a.Skv) {
+              const float bias = lc_bias_log2(lc_load_bias(
+                  a.bias, b * a.bs[0] + h * a.bs[1] + (int64_t)row * a.bs[2] + (int64_t)kj * a.bs[3],
+                  a.bias_dtype));
+              x += bias;
+              masked = bias == -INFINITY;
+            }
           }
+          const float p = lc_exp2(x);
+          s[r] = masked ? kF32Masked : p;
+          dp[r] = masked ? kF32Masked : p * (dp[r] - d4[i]);
         }
-        const float p = lc_exp2(x);
-        s[r] = masked ? kF32Masked : p;
-        dp[r] = masked ? kF32Masked : p * (dp[r] - d4[i]);
       }
-    }
+    };
+    if (BIAS || edge)
+      softmax_grad(std::true_type{});
+    else
+      softmax_grad(std::false_type{});
     lc_compiler_fence();
     float* scratch = slab + wave * 32 * (DPAD + 4);
     if ((BIAS || edge) && (oc.any_nonfinite() || qc.any_nonfinite())) {
@@ -1477,7 +1491,7 @@ int lc_prefill_attn_bwd(const void* q, const void* k, const void* v, const void*
   }
   // fp32 MFMA kernels: D a multiple of 4 up to 128, 16-byte aligned output
   // rows, one head's rows (and the zero tiles past them) within 32-bit byte
-  // offsets. At [2, 16/8, 1024, 64] 267 us against 3193 us for the lane-per-row
+  // offsets. At [2, 16/8, 1024, 64] 174 us against 3193 us for the lane-per-row
   // kernels, which keep the other head_dims.
   bool f32 = D % 4 == 0 && D <= 128 && lc_aligned(dq, 16) && lc_aligned(dk, 16) &&
              lc_aligned(dv, 16);
