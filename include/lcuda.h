@@ -266,6 +266,14 @@ LC_API int lc_decode_linear_partials(const void* x, int64_t x_row_stride, const 
                                      int64_t weight_row_stride, float* partials, int64_t M,
                                      int64_t N, int64_t K, int shares, int dtype, void* stream);
 
+/* y = x W^T in fp32 for the small inference projections of an fp32 model (the
+ * nn.Linear calls of models/llama3/attention.py:100-102,154 and mlp.py:35-43):
+ * x [M, K], w [N, K] and y [M, N], rows x/w/y_stride elements apart (>= K, K, N).
+ * N and K multiples of 4, y rows 16-byte aligned. */
+LC_API int lc_linear_f32(const float* x, int64_t x_stride, const float* w, int64_t w_stride,
+                         float* y, int64_t y_stride, int64_t M, int64_t N, int64_t K,
+                         void* stream);
+
 /* Bytes of fp32 workspace lc_paged_decode_fwd needs for these sizes
  * (partial outputs and logsumexps of every split). */
 LC_API int64_t lc_paged_decode_workspace_bytes(int64_t B, int64_t Hq, int64_t D, int64_t max_splits);

@@ -92,6 +92,10 @@ _SIGNATURES = {
         [_c_p, _c_p, _c_i64, _c_i64, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64,
          _c_i64, ctypes.c_float, ctypes.c_int, ctypes.c_int, _c_p],
     ),
+    "lc_linear_f32": (
+        ctypes.c_int,
+        [_c_p, _c_i64, _c_p, _c_i64, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_p],
+    ),
     "lc_paged_decode_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64, _c_i64]),
     "lc_paged_decode_counter_count": (_c_i64, []),
     "lc_paged_decode_fwd": (

@@ -11,6 +11,8 @@ import contextlib
 import math
 
 import torch
+import torch.nn.functional as F
+from torch.nn.modules import module as _module
 
 from llm_cuda import _native as nat
 
@@ -698,6 +700,79 @@ def decode_linear_partials(x: torch.Tensor, weight: torch.Tensor, shares: int = 
                 parts.data_ptr(), M, N, K, S, nat.lc_dtype(x), _stream(dev))
         nat.check(rc, "lc_decode_linear_partials")
     return PartialSum(parts, (*lead, N), x.dtype)
+
+
+# ---------------------------------------------------------------------------
+# Small fp32 projections  (reference: the nn.Linear calls of an fp32 model,
+# models/llama3/attention.py:100-102,154 and mlp.py:35-43)
+# ---------------------------------------------------------------------------
+def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """True where linear_f32 takes a projection over from the library's GEMM:
+    fp32 on the GPU, K <= 768, at most 256 tiles of 32 x 32 outputs, no autograd
+    graph being recorded, no autocast, and not inside torch_projections().
+
+    The line: one round of the CUs and a K that eight waves contract in a few
+    microseconds. Graph-replayed us a call, here / library: K 256, N 512, 64
+    tiles 4.5 / 5.7, 256 tiles 5.0 / 5.8, N 1376, 344 tiles 7.2 / 5.7; N 256, 64
+    tiles, K 688 6.7 / 160, K 1024 10.6 / 6.0; N 384, K 384 5.8 / 5.4 (the
+    library's call costs 13 us more on the host)."""
+    if not _NATIVE_PROJECTIONS[0] or not (x.is_cuda and weight.is_cuda):
+        return False
+    if not (x.dtype == weight.dtype == torch.float32 and weight.dim() == 2 and x.dim() >= 1):
+        return False
+    N, K = weight.shape
+    if not (0 < K <= 768 and N > 0 and K % 4 == 0 and N % 4 == 0 and x.shape[-1] == K):
+        return False
+    rows = x.numel() // K
+    if not 0 < -(-rows // 32) * -(-N // 32) <= 256:
+        return False
+    if _records_grad(x, weight) or torch.is_autocast_enabled():
+        return False
+    return weight.stride(1) == 1 and (N == 1 or K <= weight.stride(0) < 2 ** 23)
+
+
+def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """x @ weight.T in fp32 (x [..., K], weight [N, K])."""
+    if _records_grad(x, weight):
+        raise RuntimeError("linear_f32 is inference-only (autograd is recording)")
+    if x.dtype != torch.float32 or weight.dtype != torch.float32:
+        raise TypeError("linear_f32 takes fp32 tensors")
+    if weight.dim() != 2 or x.shape[-1] != weight.shape[1]:
+        raise ValueError(f"x {tuple(x.shape)} and weight {tuple(weight.shape)} do not match")
+    dev = nat.require_device(x, weight)
+    N, K = weight.shape
+    x2 = x.reshape(-1, K)
+    M = x2.shape[0]
+    if x2.stride(-1) != 1 or (M > 1 and not K <= x2.stride(0) < 2 ** 23):
+        x2 = x2.contiguous()
+    if weight.stride(-1) != 1 or (N > 1 and weight.stride(0) < K):
+        weight = weight.contiguous()
+    y = torch.empty(*x.shape[:-1], N, dtype=torch.float32, device=dev)
+    lib = nat.load()
+    with _DeviceGuard(dev):
+        rc = lib.lc_linear_f32(
+            x2.data_ptr(), x2.stride(0) if M > 1 else K, weight.data_ptr(),
+            weight.stride(0) if N > 1 else K, y.data_ptr(), N, M, N, K, _stream(dev))
+    nat.check(rc, "lc_linear_f32")
+    return y
+
+
+def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """x @ weight.T: linear_f32 where it applies, else F.linear."""
+    if linear_f32_applies(x, weight):
+        return linear_f32(x, weight)
+    return F.linear(x, weight)
+
+
+def project(x: torch.Tensor, module: torch.nn.Module) -> torch.Tensor:
+    """module(x) for a projection; a plain bias-free nn.Linear without hooks runs
+    as linear_f32 where that applies."""
+    if (type(module) is torch.nn.Linear and module.bias is None
+            and not (module._forward_hooks or module._forward_pre_hooks
+                     or _module._global_forward_hooks or _module._global_forward_pre_hooks)
+            and linear_f32_applies(x, module.weight)):
+        return linear_f32(x, module.weight)
+    return module(x)
 
 
 # ---------------------------------------------------------------------------

@@ -6,7 +6,8 @@ differs only in how the attention itself is computed, all on HIP kernels:
   * Inference projections: q, k and v come out of one GEMM against the
     concatenated weight (the parameters alias its row blocks). With at most
     32 rows (a decode step) that GEMM and o_proj are native launches that
-    stream the weight once (`decode_linear`).
+    stream the weight once (`decode_linear`); the small projections of an fp32
+    model are native too (`linear_f32`).
   * RoPE: Q and K rotated in one launch, reading the transposed projection
     views directly. The cos/sin tables are built once for a range of
     positions and sliced per call (every row depends only on its position,
@@ -32,7 +33,6 @@ from __future__ import annotations
 
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from llm_cuda.kernels import _ops
 from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
@@ -124,7 +124,7 @@ class Llama3Attention(nn.Module):
         if FusedLinearWeights.usable(self.q_proj, self.k_proj, self.v_proj):
             nq, nk, _ = self._qkv.sizes()
             w = self._qkv.weight()
-            qkv = _ops.decode_linear(x, w) if _ops.decode_linear_applies(x, w) else F.linear(x, w)
+            qkv = _ops.decode_linear(x, w) if _ops.decode_linear_applies(x, w) else _ops.linear(x, w)
             q = self._shape(qkv[..., :nq], self.num_heads)
             k = self._shape(qkv[..., nq:nq + nk], self.num_kv_heads)
             v = self._shape(qkv[..., nq + nk:], self.num_kv_heads)
@@ -165,7 +165,7 @@ class Llama3Attention(nn.Module):
                 return _ops.decode_linear_partials(out, wo), cache
             if _ops.decode_linear_applies(out, wo):
                 return _ops.decode_linear(out, wo), cache
-            return self.o_proj(out), cache
+            return _ops.project(out, self.o_proj), cache
 
         cos, sin = self._rope_tables(past_len, seq_len, x.device, x.dtype)
         q, k = apply_rotary(q, k, cos, sin)
@@ -207,5 +207,5 @@ class Llama3Attention(nn.Module):
                                                     q_offset=past_len)
 
         out = out.transpose(1, 2).reshape(bsz, seq_len, self.num_heads * self.head_dim)
-        return self.o_proj(out), present
+        return _ops.project(out, self.o_proj), present
 

@@ -9,10 +9,10 @@ takes 44 us from that layout against 52-55 us from [2N, K].
 At a decode step (at most 32 rows, bf16/f16) gate, up and the SwiGLU are one
 native launch instead (`decode_linear(swiglu=True)`): the [gate; up] weight is
 streamed once and only the SwiGLU output is written, with the same roundings.
+The small projections of an fp32 model are native as well (`linear_f32`).
 """
 import torch
 import torch.nn as nn
-import torch.nn.functional as F
 
 from llm_cuda.kernels import _ops
 from llm_cuda.kernels.triton.swiglu import triton_swiglu
@@ -50,6 +50,6 @@ class Llama3MLP(nn.Module):
                 if _ops.decode_linear_applies(h, wd):
                     return _ops.decode_linear(h, wd)
                 return self.down_proj(h)
-            gu = F.linear(x, w)
-            return self.down_proj(triton_swiglu(gu[..., :n], gu[..., n:]))
+            gu = _ops.linear(x, w)
+            return _ops.project(triton_swiglu(gu[..., :n], gu[..., n:]), self.down_proj)
         return self.down_proj(triton_swiglu(self.gate_proj(x), self.up_proj(x)))

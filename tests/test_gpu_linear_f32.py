@@ -1,0 +1,48 @@
+"""GPU parity of the small fp32 projections (lc_linear_f32) against float64: edges
+of the 32 x 32 tiles, K remainders of the 8 waves' shares, strided rows, and the
+calls the rule leaves to torch.
+
+Bound: a sum of K fp32 products, K 2^-23 of the largest value's scale.
+"""
+import pytest
+import torch
+import torch.nn.functional as F
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("M,N,K", [
+    (1, 4, 4), (2, 512, 256), (31, 36, 12), (32, 32, 64), (33, 100, 68), (128, 256, 688),
+    (65, 1376, 256), (3, 8, 768), (256, 1024, 20)])
+@pytest.mark.parametrize("strided", [False, True])
+def test_linear_f32_matches_float64(cuda, M, N, K, strided):
+    from llm_cuda.kernels import _ops
+
+    g = torch.Generator().manual_seed(M + N + K)
+    pad = 12 if strided else 0
+    x = torch.randn(M, K + pad, generator=g).to(cuda)[:, :K]
+    w = torch.randn(N, K + pad, generator=g).to(cuda)[:, :K]
+    assert _ops.linear_f32_applies(x, w)
+    y = _ops.linear_f32(x, w)
+    ref = F.linear(x.double(), w.double())
+    assert (y.double() - ref).abs().max().item() <= K * 2.0 ** -23 * max(1.0, ref.abs().max().item())
+    assert torch.equal(_ops.linear(x.view(1, M, K) if not strided else x, w).view(M, N), y)
+
+
+def test_linear_f32_leaves_other_calls_to_torch(cuda):
+    from llm_cuda.kernels import _ops
+
+    x, w = torch.randn(4, 64, device=cuda), torch.randn(32, 64, device=cuda)
+    assert _ops.linear_f32_applies(x, w)
+    assert not _ops.linear_f32_applies(x.bfloat16(), w.bfloat16())
+    assert not _ops.linear_f32_applies(x, w.requires_grad_(True))
+    w = w.detach()
+    assert not _ops.linear_f32_applies(x.expand(4096, 4, 64), w)      # too many tiles
+    assert not _ops.linear_f32_applies(x[:, :62], w[:, :62])          # K % 4
+    assert not _ops.linear_f32_applies(x, w.t().contiguous().t())     # column-major weight
+    assert not _ops.linear_f32_applies(x[:0], w)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert _ops.linear(x, w).dtype == torch.bfloat16
+    lin = torch.nn.Linear(64, 32, bias=False, device=cuda).requires_grad_(False)
+    lin.register_forward_hook(lambda m, i, o: o + 1)
+    assert torch.equal(_ops.project(x, lin), F.linear(x, lin.weight) + 1)
