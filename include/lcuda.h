@@ -149,6 +149,24 @@ LC_API int lc_prefill_attn_fwd(const void* q, const void* k, const void* v, void
                         const void* bias, const int64_t* bias_strides, int bias_dtype,
                         int32_t* counters, float scale, int dtype, void* stream);
 
+/* lc_prefill_attn_fwd with a workspace: where an unmasked bf16/f16 call has too
+ * few row groups to fill the device (a short chunk over a long cached prefix),
+ * each row group's keys are split into ranges computed side by side, whose fp32
+ * partial outputs and logsumexps go through the workspace and are merged by a
+ * second launch. lc_prefill_attn_workspace_bytes: what such a call needs (0:
+ * the call is not split); with less, or NULL, the call runs unsplit. 16-byte
+ * aligned; calls that may overlap need their own. */
+LC_API int64_t lc_prefill_attn_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                               int64_t Skv, int64_t D, int64_t q_offset,
+                                               int has_bias, int dtype);
+LC_API int lc_prefill_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                                  int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv,
+                                  int64_t D, const int64_t* q_strides, const int64_t* k_strides,
+                                  const int64_t* v_strides, const int64_t* o_strides,
+                                  int64_t q_offset, const void* bias, const int64_t* bias_strides,
+                                  int bias_dtype, int32_t* counters, void* workspace,
+                                  int64_t workspace_bytes, float scale, int dtype, void* stream);
+
 /* Bytes of workspace lc_prefill_attn_bwd needs: two fp32 values per query row
  * (delta = rowsum(dO*O), and lse * log2(e)). */
 LC_API int64_t lc_prefill_attn_bwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq);

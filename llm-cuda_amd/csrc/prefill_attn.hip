@@ -45,6 +45,12 @@ struct PrefillArgs {
   // out through it; dyn_light == 0: every workgroup's item from its block id.
   int* ticket;
   int dyn_units, dyn_light;
+  // Key splits (the SPLIT instances): n_splits ranges of split_tiles 64-key
+  // tiles each; range z writes its normalised fp32 output to
+  // ws_o[z][(b, h, i)][D] and its base-2 logsumexp to ws_l[z][(b, h, i)].
+  float* ws_o;
+  float* ws_l;
+  int n_splits, split_tiles;
 };
 
 // ---------------------------------------------------------------------------
@@ -321,7 +327,12 @@ constexpr int kPrefillCounterInts = 64;
 // With an additive bias (BIAS != 0) the kernel runs one wave per SIMD: the
 // bias tile held one iteration ahead does not fit the two-wave register
 // budget without spills.
-template <typename T, int DPAD, int BIAS>
+//
+// SPLIT: one workgroup computes one key range of a row group (see
+// prefill_merge_kernel); the range's first key becomes key 0, so the keys
+// before it are out of sight and the causal offset shrinks with it (below zero
+// for rows that see none of the range).
+template <typename T, int DPAD, int BIAS, bool SPLIT = false>
 __global__ __launch_bounds__(64 * kPfWaves) __attribute__((
     amdgpu_waves_per_eu(BIAS == 0 ? 2 : 1, BIAS == 0 ? 2 : 1))) void
 prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
@@ -406,6 +417,19 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   unit = __builtin_amdgcn_readfirstlane(unit);
   rbg = __builtin_amdgcn_readfirstlane(rbg);
   asm volatile("" : "+s"(unit), "+s"(rbg));
+  int64_t split_row = 0;  // this split's first row of ws_o / ws_l
+  if constexpr (SPLIT) {
+    // A unit's splits follow one another, so a range's row groups, which read
+    // the same keys, run on one XCD.
+    const int z = unit % a.n_splits;
+    unit /= a.n_splits;
+    const int64_t k0 = (int64_t)z * a.split_tiles * kPfKeys;
+    a.k = static_cast<const T*>(a.k) + k0 * a.ks[2];
+    a.v = static_cast<const T*>(a.v) + k0 * a.vs[2];
+    a.Skv = static_cast<int>(min(a.Skv - k0, (int64_t)a.split_tiles * kPfKeys));
+    a.q_offset -= static_cast<int>(k0);
+    split_row = (int64_t)z * a.B * a.Hq * a.Sq;
+  }
   const int kvh_hg = unit % (a.Hkv * n_hg);
   const int b = unit / (a.Hkv * n_hg);
   const int kvh = kvh_hg / n_hg;
@@ -814,6 +838,27 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   float l_tot = l_lane + __shfl_xor(l_lane, 32, 64);
   if (qi >= a.Sq) return;
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
+  if constexpr (SPLIT) {
+    // (the merge reads no output of a range without visible keys)
+    const int64_t row = split_row + ((int64_t)b * a.Hq + head) * a.Sq + qi;
+    float* prow = a.ws_o + row * a.D;
+    if (l_tot > 0.f) {
+#pragma unroll
+      for (int dt = 0; dt < DTL; ++dt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int d = dt * 32 + j * 8 + hh * 4;
+          if (d < a.D) {
+            f32x4_t w;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = o[dt][j * 4 + i] * inv;
+            *reinterpret_cast<f32x4_t*>(prow + d) = w;
+          }
+        }
+    }
+    if (hh == 0) a.ws_l[row] = l_tot > 0.f ? m_ref + lc_log2(l_tot) : -INFINITY;
+    return;
+  }
   T* orow = static_cast<T*>(a.o) + b * a.os[0] + (int64_t)head * a.os[1] + (int64_t)qi * a.os[2];
 #pragma unroll
   for (int dt = 0; dt < DTL; ++dt)
@@ -833,6 +878,44 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
         l_tot > 0.f ? (m_ref + lc_log2(l_tot)) * kLn2 : -INFINITY;
 }
 
+// Combines the key ranges of SPLIT launches: o = sum_z 2^(l_z - L) o_z with
+// L = log2 sum_z 2^(l_z). D / 4 lanes a row, 16 bytes of each range per lane;
+// bound by reading the fp32 partials once (they are mostly still in L2).
+template <typename T>
+__global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int64_t rows) {
+  const int lpr = a.D / 4;  // lanes per row
+  const int rpb = 256 / lpr;
+  const int sub = threadIdx.x / lpr;
+  const int64_t row = (int64_t)blockIdx.x * rpb + sub;
+  if (sub >= rpb || row >= rows) return;
+  const int d = (threadIdx.x - sub * lpr) * 4;
+  float m = -INFINITY;
+  for (int z = 0; z < a.n_splits; ++z) m = fmaxf(m, a.ws_l[z * rows + row]);
+  float l = 0.f;
+  f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
+  if (m != -INFINITY) {
+    for (int z = 0; z < a.n_splits; ++z) {
+      const float lz = a.ws_l[z * rows + row];
+      if (lz == -INFINITY) continue;  // no visible key: nothing was written
+      const float w = lc_exp2(lz - m);
+      l += w;
+      acc += *reinterpret_cast<const f32x4_t*>(a.ws_o + (z * rows + row) * a.D + d) * w;
+    }
+  }
+  const float inv = l > 0.f ? 1.0f / l : 0.f;
+  const int i = static_cast<int>(row % a.Sq);
+  const int64_t bh = row / a.Sq;
+  const int h = static_cast<int>(bh % a.Hq);
+  const int64_t b = bh / a.Hq;
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  t4 out;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) out[e] = lc_from_f32<T>(acc[e] * inv);
+  *reinterpret_cast<t4*>(static_cast<T*>(a.o) + b * a.os[0] + h * a.os[1] +
+                         (int64_t)i * a.os[2] + d) = out;
+  if (a.lse != nullptr && d == 0) a.lse[row] = l > 0.f ? (m + lc_log2(l)) * kLn2 : -INFINITY;
+}
+
 static int gcd_int(int x, int y) {
   while (y) {
     const int t = x % y;
@@ -850,14 +933,70 @@ void launch_mfma_bias(const PrefillArgs& a, dim3 grid, int hw, int n_rbg, hipStr
     prefill_mfma_kernel<T, 128, BIAS><<<grid, 64 * kPfWaves, 0, st>>>(a, hw, n_rbg);
 }
 
+// Row groups of a (batch, kv head, head group) unit, and their number in all.
+struct PfGrid {
+  int hw, n_rbg;
+  int64_t nwg;
+};
+PfGrid pf_grid(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq) {
+  const int G = static_cast<int>(Hq / Hkv), hw = gcd_int(G, kPfWaves), rbw = kPfWaves / hw;
+  const int64_t n_rb = (Sq + kPfRows - 1) / kPfRows, n_rbg = (n_rb + rbw - 1) / rbw;
+  return {hw, static_cast<int>(n_rbg), n_rbg * Hkv * (G / hw) * B};
+}
+
+// Key splits of an unmasked MFMA call (1: none). A grid that leaves at least
+// half of the CUs without a workgroup is split into as many ranges as give each
+// CU one, of at least 8 tiles; a second workgroup on a CU shares its matrix
+// cores, so it gains less than the ranges' starts and the merge (a launch and
+// an fp32 pass over the partials) cost. us a call at D 128, 32/8 heads, unsplit
+// / split: 128 x 4224 keys (32 workgroups) 66.6 / 30.7 at 8 ranges; 512 x 8192
+// (128) 121 / 82 at 2, 81 at 4; 256 x 2304 (64) 39.6 / 30.4 at 4; 1000 x 5000
+// (256) 86.9 / 93.9 at 2. Under 32 tiles the merge costs more than the shorter
+// chain saves (128 x 1152: 24.1 / 26.6 at 2, 512 x 1536: 30.8 / 33.4).
+constexpr int kSplitMinTiles = 32, kSplitTiles = 8;
+int pf_splits(const PfGrid& g, int64_t Sq, int64_t Skv, int64_t q_offset) {
+  const int64_t keys = Skv < Sq + q_offset ? Skv : Sq + q_offset;
+  const int64_t tiles = (keys + kPfKeys - 1) / kPfKeys;
+  if (g.nwg <= 0 || tiles < kSplitMinTiles) return 1;
+  const int64_t z = lc_cu_count() / g.nwg, most = tiles / kSplitTiles;
+  return static_cast<int>(z < 2 ? 1 : z < most ? z : most);
+}
+int64_t pf_split_bytes(int64_t rows, int64_t D, int z) {
+  return z < 2 ? 0 : z * rows * (D + 1) * 4;
+}
+
 template <typename T>
-int launch_mfma(const PrefillArgs& a, hipStream_t st) {
-  const int hw = gcd_int(a.G, kPfWaves);
-  const int rbw = kPfWaves / hw;
-  const int n_rb = (a.Sq + kPfRows - 1) / kPfRows;
-  const int n_rbg = (n_rb + rbw - 1) / rbw;
-  const int64_t nwg = (int64_t)n_rbg * a.Hkv * (a.G / hw) * a.B;
+int launch_mfma_split(PrefillArgs a, const PfGrid& g, int z, hipStream_t st) {
+  const int64_t keys = (int64_t)a.Sq + a.q_offset < a.Skv ? (int64_t)a.Sq + a.q_offset : a.Skv;
+  const int64_t tiles = (keys + kPfKeys - 1) / kPfKeys;
+  a.split_tiles = static_cast<int>((tiles + z - 1) / z);
+  a.n_splits = static_cast<int>((tiles + a.split_tiles - 1) / a.split_tiles);
+  const int64_t rows = (int64_t)a.B * a.Hq * a.Sq;
+  a.ws_l = a.ws_o + z * rows * a.D;
+  const int64_t nwg = g.nwg * a.n_splits;
+  const int rpb = 256 / (a.D / 4);
+  const int64_t mwg = (rows + rpb - 1) / rpb;
+  LC_REQUIRE(nwg < (1LL << 31) && mwg < (1LL << 31), "lc_prefill_attn_fwd: grid too large");
+  const unsigned n = static_cast<unsigned>(nwg);
+  if (a.D <= 64)
+    prefill_mfma_kernel<T, 64, 0, true><<<n, 64 * kPfWaves, 0, st>>>(a, g.hw, g.n_rbg);
+  else
+    prefill_mfma_kernel<T, 128, 0, true><<<n, 64 * kPfWaves, 0, st>>>(a, g.hw, g.n_rbg);
+  prefill_merge_kernel<T><<<static_cast<unsigned>(mwg), 256, 0, st>>>(a, rows);
+  return lc_check_launch("lc_prefill_attn_fwd (split)");
+}
+
+template <typename T>
+int launch_mfma(const PrefillArgs& a, int64_t ws_bytes, hipStream_t st) {
+  const PfGrid g = pf_grid(a.B, a.Hq, a.Hkv, a.Sq);
+  const int hw = g.hw, n_rbg = g.n_rbg;
+  const int64_t nwg = g.nwg;
   LC_REQUIRE(nwg < (1LL << 31), "lc_prefill_attn_fwd: grid too large");
+  if (a.bias == nullptr && a.ws_o != nullptr) {
+    const int z = pf_splits(g, a.Sq, a.Skv, a.q_offset);
+    if (z > 1 && ws_bytes >= pf_split_bytes((int64_t)a.B * a.Hq * a.Sq, a.D, z))
+      return launch_mfma_split<T>(a, g, z, st);
+  }
   dim3 grid(static_cast<unsigned>(nwg));
   // Dynamic tail: with a ticket, no bias, whole units per XCD (units a
   // multiple of 8), >= 8 row groups per unit and more than two rounds of
@@ -924,12 +1063,34 @@ extern "C" {
 
 int64_t lc_prefill_attn_counter_count(void) { return kPrefillCounterInts; }
 
+int64_t lc_prefill_attn_workspace_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                        int64_t Skv, int64_t D, int64_t q_offset, int has_bias,
+                                        int dtype) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Sq <= 0 || Skv <= 0 || D <= 0 ||
+      q_offset < 0 || has_bias || dtype == LC_DTYPE_F32 || D % 8 != 0 || D > 128)
+    return 0;
+  return pf_split_bytes(B * Hq * Sq, D, pf_splits(pf_grid(B, Hq, Hkv, Sq), Sq, Skv, q_offset));
+}
+
 int lc_prefill_attn_fwd(const void* q, const void* k, const void* v, void* o, float* lse,
                         int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv, int64_t D,
                         const int64_t* q_strides, const int64_t* k_strides,
                         const int64_t* v_strides, const int64_t* o_strides, int64_t q_offset,
                         const void* bias, const int64_t* bias_strides, int bias_dtype,
                         int32_t* counters, float scale, int dtype, void* stream) {
+  return lc_prefill_attn_fwd_ws(q, k, v, o, lse, B, Hq, Hkv, Sq, Skv, D, q_strides, k_strides,
+                                v_strides, o_strides, q_offset, bias, bias_strides, bias_dtype,
+                                counters, nullptr, 0, scale, dtype, stream);
+}
+
+int lc_prefill_attn_fwd_ws(const void* q, const void* k, const void* v, void* o, float* lse,
+                           int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq, int64_t Skv, int64_t D,
+                           const int64_t* q_strides, const int64_t* k_strides,
+                           const int64_t* v_strides, const int64_t* o_strides, int64_t q_offset,
+                           const void* bias, const int64_t* bias_strides, int bias_dtype,
+                           int32_t* counters, void* workspace, int64_t workspace_bytes,
+                           float scale, int dtype, void* stream) {
+  LC_REQUIRE(lc_aligned(workspace, 16), "lc_prefill_attn_fwd: workspace not 16-byte aligned");
   LC_REQUIRE(q_strides && k_strides && v_strides && o_strides,
              "lc_prefill_attn_fwd: null stride array");
   LC_REQUIRE(lc_aligned(counters, 4), "lc_prefill_attn_fwd: counters not 4-byte aligned");
@@ -980,6 +1141,7 @@ int lc_prefill_attn_fwd(const void* q, const void* k, const void* v, void* o, fl
   a.bias = Skv > 0 ? bias : nullptr;
   a.bias_dtype = bias_dtype;
   a.ticket = counters;
+  a.ws_o = static_cast<float*>(workspace);
   if (bias != nullptr)
     for (int i = 0; i < 4; ++i) a.bs[i] = bias_strides[i];
   hipStream_t st = lc_stream(stream);
@@ -1020,9 +1182,9 @@ int lc_prefill_attn_fwd(const void* q, const void* k, const void* v, void* o, fl
     case LC_DTYPE_F32:
       return f32 ? launch_f32(a, st) : launch_generic<float>(a, st);
     case LC_DTYPE_BF16:
-      return mfma ? launch_mfma<bf16_t>(a, st) : launch_generic<bf16_t>(a, st);
+      return mfma ? launch_mfma<bf16_t>(a, workspace_bytes, st) : launch_generic<bf16_t>(a, st);
     case LC_DTYPE_F16:
-      return mfma ? launch_mfma<f16_t>(a, st) : launch_generic<f16_t>(a, st);
+      return mfma ? launch_mfma<f16_t>(a, workspace_bytes, st) : launch_generic<f16_t>(a, st);
     default:
       return lc_fail(LC_EINVAL, "lc_prefill_attn_fwd: unknown dtype %d", dtype);
   }

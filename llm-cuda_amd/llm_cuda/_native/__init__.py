@@ -60,6 +60,16 @@ _SIGNATURES = {
          _c_i64p, _c_i64p, _c_i64p, _c_i64, _c_p, _c_i64p, ctypes.c_int, _c_p, ctypes.c_float,
          ctypes.c_int, _c_p],
     ),
+    "lc_prefill_attn_workspace_bytes": (
+        _c_i64,
+        [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int, ctypes.c_int],
+    ),
+    "lc_prefill_attn_fwd_ws": (
+        ctypes.c_int,
+        [_c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64p,
+         _c_i64p, _c_i64p, _c_i64p, _c_i64, _c_p, _c_i64p, ctypes.c_int, _c_p, _c_p, _c_i64,
+         ctypes.c_float, ctypes.c_int, _c_p],
+    ),
     "lc_prefill_attn_bwd_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
     "lc_prefill_attn_bwd": (
         ctypes.c_int,

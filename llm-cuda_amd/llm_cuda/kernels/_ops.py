@@ -387,17 +387,26 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_offse
     # any eager call runs the static order (no counters).
     counters = _zeroed_counters("prefill", dev, lib.lc_prefill_attn_counter_count(),
                                 optional=True)
+    # Fp32 partials of a call whose keys are split (the library splits no call
+    # of under 32 tiles of 64 visible keys; 0 bytes: it does not split this one).
+    ws, ws_bytes = None, 0
+    if bias is None and Skv > 1984 and Sq + q_offset > 1984:
+        ws_bytes = lib.lc_prefill_attn_workspace_bytes(B, Hq, Hkv, Sq, Skv, D, int(q_offset), 0,
+                                                       nat.lc_dtype(q))
+        if ws_bytes > 0:
+            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
     with _DeviceGuard(dev):
-        rc = lib.lc_prefill_attn_fwd(
+        rc = lib.lc_prefill_attn_fwd_ws(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
             None if lse is None else lse.data_ptr(), B, Hq, Hkv, Sq, Skv, D,
             _i64arr(q.stride()), _i64arr(k.stride()), _i64arr(v.stride()), _i64arr(out.stride()),
             int(q_offset), None if bias is None else bias.data_ptr(),
             None if bias is None else _i64arr(bias.stride()),
             0 if bias is None else nat.lc_dtype(bias),
-            None if counters is None else counters.data_ptr(), float(scale), nat.lc_dtype(q),
+            None if counters is None else counters.data_ptr(),
+            None if ws is None else ws.data_ptr(), ws_bytes, float(scale), nat.lc_dtype(q),
             _stream(dev))
-    nat.check(rc, "lc_prefill_attn_fwd")
+    nat.check(rc, "lc_prefill_attn_fwd_ws")
     return (out, lse) if return_lse else out
 
 
