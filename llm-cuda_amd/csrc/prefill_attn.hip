@@ -321,12 +321,19 @@ constexpr int kPfWaves = 4;
 constexpr int kPfRows = 32;     // query rows per wave
 constexpr int kPfKeys = 64;     // keys per tile
 constexpr float kPfRescaleLog2 = 8.0f;
+constexpr int kPfKeyBias = 4096;  // keys of a key bias that LDS holds (16 KB)
+constexpr int pf_waves_per_simd(int bias) { return bias == 0 || bias == 3 ? 2 : 1; }
 // int32 counters lc_prefill_attn_fwd takes: the dynamic tail's ticket, padded to 256 bytes.
 constexpr int kPrefillCounterInts = 64;
 
-// With an additive bias (BIAS != 0) the kernel runs one wave per SIMD: the
-// bias tile held one iteration ahead does not fit the two-wave register
-// budget without spills.
+// BIAS: 0 none, 1 in dtype T, 2 in fp32, 3 a key bias. With a bias per query row
+// (1, 2) the kernel runs one wave per SIMD: the bias tile held one iteration
+// ahead does not fit the two-wave register budget without spills. A bias alike
+// for every query row and head (the [B, 1, 1, Skv] padding masks) is staged in
+// LDS at the start, divided by scale_log2, and the S^T accumulators start from
+// it instead of from zero: no registers, no instructions per score, so it runs
+// two waves per SIMD. [8, 32/8, 1000, 128] with a padding mask: 108 us as 3,
+// 194 us as 1, 107 us unmasked.
 //
 // SPLIT: one workgroup computes one key range of a row group (see
 // prefill_merge_kernel); the range's first key becomes key 0, so the keys
@@ -334,7 +341,7 @@ constexpr int kPrefillCounterInts = 64;
 // for rows that see none of the range).
 template <typename T, int DPAD, int BIAS, bool SPLIT = false>
 __global__ __launch_bounds__(64 * kPfWaves) __attribute__((
-    amdgpu_waves_per_eu(BIAS == 0 ? 2 : 1, BIAS == 0 ? 2 : 1))) void
+    amdgpu_waves_per_eu(pf_waves_per_simd(BIAS), pf_waves_per_simd(BIAS)))) void
 prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   typedef Mfma32<T> Ops;
   typedef typename Ops::v8 v8;
@@ -455,21 +462,31 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   // descriptor; the tile's values are loaded one iteration ahead of the SM1
   // that adds them (see BiasTile).
   const int qi = r0 + l32;
+  constexpr bool ROW_BIAS = BIAS == 1 || BIAS == 2;
   constexpr int besz = BIAS == 2 ? 4 : 2;
-  BiasTile<T, BIAS == 0 ? 1 : BIAS> btile;
+  BiasTile<T, ROW_BIAS ? BIAS : 1> btile;
   const __amdgpu_buffer_rsrc_t brs = __builtin_amdgcn_make_buffer_rsrc(
-      const_cast<char*>(static_cast<const char*>(BIAS != 0 ? a.bias : a.q) +
-                        (BIAS != 0 ? (b * a.bs[0] + (int64_t)head * a.bs[1]) * besz : 0)),
+      const_cast<char*>(static_cast<const char*>(ROW_BIAS ? a.bias : a.q) +
+                        (ROW_BIAS ? (b * a.bs[0] + (int64_t)head * a.bs[1]) * besz : 0)),
       0,
-      BIAS != 0 ? static_cast<int>(((int64_t)(a.Sq - 1) * a.bs[2] +
+      ROW_BIAS ? static_cast<int>(((int64_t)(a.Sq - 1) * a.bs[2] +
                                      (int64_t)(a.Skv - 1) * a.bs[3] + 1) * besz)
                 : 0,
       0x00020000);
   const int brow_b = static_cast<int>((int64_t)qi * a.bs[2] * besz);
   const int bs3_b = static_cast<int>(a.bs[3] * besz);
   auto load_bias = [&](int t) __attribute__((always_inline)) {
-    if constexpr (BIAS != 0) btile.load(brs, brow_b, t * kPfKeys, hh, bs3_b, a.bias_vec != 0);
+    if constexpr (ROW_BIAS) btile.load(brs, brow_b, t * kPfKeys, hh, bs3_b, a.bias_vec != 0);
   };
+  __shared__ __align__(16) float key_bias[BIAS == 3 ? kPfKeyBias : 4];
+  if constexpr (BIAS == 3) {
+    // (the host passes at most kPfKeyBias visible keys; published by the barrier
+    // before the first scores)
+    const float inv = 1.0f / a.scale_log2;
+    for (int k = tid; k < kv_end; k += 64 * kPfWaves)
+      key_bias[k] =
+          lc_bias_log2(lc_load_bias(a.bias, b * a.bs[0] + k * a.bs[3], a.bias_dtype)) * inv;
+  }
 
   // Q^T operand registers.
   v8 qop[KS];
@@ -546,11 +563,23 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
     return wave_active && t < n_tiles && t * kPfKeys < my_kv_end;
   };
 
-  auto qk = [&](LC_LDS const char* kt_lds) __attribute__((always_inline)) {
+  auto qk = [&](LC_LDS const char* kt_lds, int k0) __attribute__((always_inline)) {
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) snx[kt][r] = 0.f;
+    if constexpr (BIAS == 3) {
+      // (what keys past kv_end read is masked)
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const f32x4_t b4 = *reinterpret_cast<LC_LDS const f32x4_t*>(
+              (LC_LDS const float*)key_bias + k0 + kt * 32 + j * 8 + hh * 4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) snx[kt][j * 4 + i] = b4[i];
+        }
+    }
     // The two 32-key halves alternate, so consecutive MFMAs are independent.
 #pragma unroll
     for (int s = 0; s < KS; ++s)
@@ -578,7 +607,15 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   // SM1 of the tile whose raw scores are in snx (keys k0 ..): sets xcu, the
   // running max and row sum; a required rescale of O is left to apply_rescale.
   auto sm1 = [&](int k0, auto mask_c) __attribute__((always_inline)) {
-    if constexpr (BIAS != 0) {
+    // (no fused s * scale - m: at a masked row's m of -1e30 its one rounding
+    // differs from m's by far more than 1)
+#pragma clang fp contract(off)
+    if constexpr (BIAS == 3) {
+#pragma unroll
+      for (int kt = 0; kt < 2; ++kt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) snx[kt][r] *= a.scale_log2;
+    } else if constexpr (BIAS != 0) {
       // Scores with the bias, in the exp2 domain.
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
@@ -728,7 +765,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
     if constexpr (BIAS == 0) {
       if (cur && nxt) {
         constexpr int NQ = 2 * KS, NP = 4 * DTL, LA = 4;
-        qk(kbuf(other));
+        qk(kbuf(other), k1);
         sm2l();
         __builtin_amdgcn_sched_group_barrier(0x100, LA, 0);
 #pragma unroll
@@ -748,7 +785,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
           __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
         }
       } else {
-        if (nxt) qk(kbuf(other));
+        if (nxt) qk(kbuf(other), k1);
         if (cur) {
           sm2l();
           check_fix();
@@ -760,7 +797,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
       return;
     }
     if (cur && nxt) {
-      qk(kbuf(other));
+      qk(kbuf(other), k1);
       sm2();
       pv(vbuf(par_c));
       sm1(k1, mask_c);
@@ -768,7 +805,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
       // SM2 VALU work; part B: 16 PV MFMAs, each with two V^T reads ahead
       // and SM1 VALU work.
       constexpr int NQ = 2 * KS, NP = 4 * DTL, LA = 4;
-      __builtin_amdgcn_sched_group_barrier(0x100, LA, 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, LA + (BIAS == 3 ? 8 : 0), 0);
 #pragma unroll
       for (int j = 0; j < NQ + NP; ++j) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -780,7 +817,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
         __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
       }
     } else {
-      if (nxt) qk(kbuf(other));
+      if (nxt) qk(kbuf(other), k1);
       if (cur) {
         sm2();
         pv(vbuf(par_c));
@@ -804,7 +841,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   if (live(0)) load_bias(0);
   pf_barrier<true>();
   if (live(0)) {
-    qk(kbuf(std::integral_constant<int, 0>{}));
+    qk(kbuf(std::integral_constant<int, 0>{}), 0);
     sm1(0, std::true_type{});
     rescale = false;  // O is still zero
   }
@@ -1015,6 +1052,12 @@ int launch_mfma(const PrefillArgs& a, int64_t ws_bytes, hipStream_t st) {
     launch_mfma_bias<T, 0>(d, dim3(static_cast<unsigned>(nwg + spare)), hw, n_rbg, st);
   } else if (a.bias == nullptr)
     launch_mfma_bias<T, 0>(a, grid, hw, n_rbg, st);
+  else if (a.bs[1] == 0 && a.bs[2] == 0 && (int64_t)a.Sq + a.q_offset < (1LL << 31) &&
+           min(a.Skv, a.Sq + a.q_offset) <= kPfKeyBias && a.scale_log2 > 1e-6f &&
+           a.scale_log2 < 1e6f)
+    // A key bias (see the kernel); a scale that its division cannot take, or
+    // more keys than LDS holds, leaves it to the row-bias instances.
+    launch_mfma_bias<T, 3>(a, grid, hw, n_rbg, st);
   else if (a.bias_dtype == LC_DTYPE_F32)
     launch_mfma_bias<T, 2>(a, grid, hw, n_rbg, st);
   else

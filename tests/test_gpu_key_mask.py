@@ -1,0 +1,80 @@
+"""GPU parity of key masks ([B, 1, 1, Skv]: staged in LDS, added through the score
+accumulators) against float64 and against the same mask written out per row
+([B, 1, Sq, Skv], the row-bias kernel): padding values of every usual size, mixed
+ones, rows with no real key and with no key at all, odd lengths, a cached prefix,
+and the most keys LDS holds with the first count past it.
+"""
+import math
+
+import pytest
+import torch
+
+from helpers import ATOL
+
+pytestmark = pytest.mark.gpu
+
+
+def _mask(kind, B, Skv, dtype, g):
+    m = torch.zeros(B, 1, 1, Skv)
+    n = max(1, Skv // 3)
+    if kind == "mixed":  # ordinary biases, -1e4, -1e9, the type's lowest and -inf
+        m = 2.0 * torch.randn(m.shape, generator=g)
+        m[..., 1::5], m[..., 2::7] = -1e4, -1e9
+        m[..., 3::11], m[..., 4::13] = torch.finfo(dtype).min, -math.inf
+    else:
+        m[0, ..., :n] = {"min": torch.finfo(dtype).min, "1e4": -1e4, "1e9": -1e9,
+                         "inf": -math.inf}[kind]
+    return m.to(dtype)
+
+
+def _reference(q, k, v, mask, off):
+    g = q.shape[1] // k.shape[1]
+    s = q.double() @ k.double().repeat_interleave(g, 1).transpose(-1, -2) / math.sqrt(q.shape[-1])
+    # (masks below -1e30 act as -1e30; the scores next to them vanish as in fp32)
+    s = (s + mask.double().clamp(min=-1e30)).masked_fill(mask.double() == -math.inf, -math.inf)
+    Sq, Skv = s.shape[-2:]
+    seen = (torch.arange(Skv, device=q.device)
+            <= torch.arange(Sq, device=q.device).view(-1, 1) + off)
+    s = s.masked_fill(~seen, -math.inf)
+    p = torch.softmax(s, -1)
+    return torch.nan_to_num(p, nan=0.0) @ v.double().repeat_interleave(g, 1)
+
+
+@pytest.mark.parametrize("kind", ["min", "1e4", "1e9", "inf", "mixed"])
+@pytest.mark.parametrize("Sq,Skv,D,dtype,mdt", [
+    (200, 200, 128, torch.bfloat16, torch.bfloat16),
+    (77, 133, 64, torch.float16, torch.float32),
+    (1, 65, 128, torch.bfloat16, torch.float32),
+])
+def test_key_mask(cuda, kind, Sq, Skv, D, dtype, mdt):
+    from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
+
+    B, Hq, Hkv, off = 2, 8, 2, Skv - Sq
+    g = torch.Generator().manual_seed(Skv)
+    q, k, v = (torch.randn(s, generator=g).to(dtype).to(cuda) for s in (
+        (B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)))
+    mask = _mask(kind, B, Skv, mdt, g).to(cuda)
+    out, lse = triton_fused_causal_attention(q, k, v, mask, return_lse=True, q_offset=off)
+    rows, rlse = triton_fused_causal_attention(
+        q, k, v, mask.expand(B, 1, Sq, Skv).contiguous(), return_lse=True, q_offset=off)
+    assert (out.float() - rows.float()).abs().max().item() <= ATOL[dtype]
+    assert torch.equal(torch.isinf(lse), torch.isinf(rlse))
+    real = torch.isfinite(lse)
+    # the two add the bias before and after the scale: a few ulp of their lse
+    assert ((lse - rlse)[real].abs() <= 1e-5 + 2.0 ** -21 * rlse[real].abs()).all()
+    if kind != "1e9" and kind != "mixed":  # (at -1e9 the fp32 scores keep a few bits)
+        assert (out.double() - _reference(q, k, v, mask, off)).abs().max().item() <= ATOL[dtype]
+
+
+@pytest.mark.parametrize("Skv", [4096, 4097])
+def test_key_mask_at_the_most_keys_staged(cuda, Skv):
+    from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
+
+    B, Hq, Hkv, Sq, D, dtype = 1, 4, 1, 40, 128, torch.bfloat16
+    g = torch.Generator().manual_seed(Skv)
+    q, k, v = (torch.randn(s, generator=g).to(dtype).to(cuda) for s in (
+        (B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)))
+    mask = _mask("min", B, Skv, dtype, g).to(cuda)
+    out = triton_fused_causal_attention(q, k, v, mask, q_offset=Skv - Sq)
+    ref = _reference(q, k, v, mask, Skv - Sq)
+    assert (out.double() - ref).abs().max().item() <= ATOL[dtype]
