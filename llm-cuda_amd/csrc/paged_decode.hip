@@ -268,10 +268,14 @@ __device__ __forceinline__ void load_q(const DecodeArgs& a, int b, int h, int h_
 // first step's K/V loads are issued (a place for arithmetic on the loaded
 // operands that should not hold up that issue). HB: the call carries an
 // additive bias (loaded with the step's K/V, one step ahead).
+// P16: pages of 16 tokens: a step's two halves are a page each, so it has two
+// page lookups and two descriptor pairs and is otherwise the same (its load instructions never
+// straddle the halves: a row group of an instruction divides 16).
 // PRE: the caller has loaded a 64-page window of the sequence's block-table
 // row that covers the range (entry window_base + lane per lane, -1 past the
 // row) and passes it as row_entry, so no table load is issued here.
-template <typename T, int DPAD, bool HB, bool PRE = false, typename QLoad, typename QFinish>
+template <typename T, int DPAD, bool HB, bool PRE = false, bool P16 = false, typename QLoad,
+          typename QFinish>
 __device__ __forceinline__ void rows_range(const DecodeArgs& a, int b, int kvh, int h,
                                            bool head_ok, int t_begin, int t_end, QLoad load_q,
                                            QFinish finish_q, T* lds_k, T* lds_v,
@@ -322,34 +326,42 @@ __device__ __forceinline__ void rows_range(const DecodeArgs& a, int b, int kvh, 
   // Issue the loads of the step starting at t. Past the range end (the
   // prefetch after the last step) every offset is out of range: zeros, no
   // memory traffic, and no branch for the wait-count bookkeeping to merge.
-  auto issue = [&](int t) -> bool {
-    const int page_idx = a.p_shift >= 0 ? (t >> a.p_shift) : (t / a.P);
-    const int slot0 = t - page_idx * a.P;
-    const bool in_split = t < t_end;
-    const int phys = __builtin_amdgcn_readlane(my_page, in_split ? page_idx - first_page : 0);
-    const bool pvalid =
-        in_split && static_cast<unsigned>(phys) < static_cast<unsigned>(a.num_pages);
-    const int64_t base = pvalid ? (int64_t)phys * a.s_page + (int64_t)kvh * a.s_head : 0;
-    const int nbytes =
-        pvalid ? static_cast<int>(((int64_t)(a.P - 1) * a.s_tok + a.D) * sizeof(T)) : 0;
-    const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(static_cast<const T*>(a.kp) + base), 0, nbytes, kBufferWord3);
-    const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<T*>(static_cast<const T*>(a.vp) + base), 0, nbytes, kBufferWord3);
+  // The result's bit gi: the page of the step's tokens gi * 16 .. + 15 is valid.
+  auto issue = [&](int t) -> int {
+    constexpr int NH = P16 ? 2 : 1;  // pages per step
+    int valid = 0;
 #pragma unroll
-    for (int i = 0; i < NI; ++i) {
-      const int row = i * RPI + srow;
-      const bool live = pvalid && t + row < t_end && chunk_in_d;
-      const int off =
-          live ? static_cast<int>(((int64_t)(slot0 + row) * a.s_tok + schunk * 8) * sizeof(T))
-               : -16;
-      sk[i] = __builtin_amdgcn_raw_buffer_load_b128(rK, off, 0, kLoadNT);
-      sv[i] = __builtin_amdgcn_raw_buffer_load_b128(rV, off, 0, kLoadNT);
+    for (int half = 0; half < NH; ++half) {
+      const int th = t + half * (kStep / NH);
+      const int page_idx = a.p_shift >= 0 ? (th >> a.p_shift) : (th / a.P);
+      const int slot0 = th - page_idx * a.P;
+      const bool in_split = th < t_end;
+      const int phys = __builtin_amdgcn_readlane(my_page, in_split ? page_idx - first_page : 0);
+      const bool pvalid =
+          in_split && static_cast<unsigned>(phys) < static_cast<unsigned>(a.num_pages);
+      const int64_t base = pvalid ? (int64_t)phys * a.s_page + (int64_t)kvh * a.s_head : 0;
+      const int nbytes =
+          pvalid ? static_cast<int>(((int64_t)(a.P - 1) * a.s_tok + a.D) * sizeof(T)) : 0;
+      const __amdgpu_buffer_rsrc_t rK = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<T*>(static_cast<const T*>(a.kp) + base), 0, nbytes, kBufferWord3);
+      const __amdgpu_buffer_rsrc_t rV = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<T*>(static_cast<const T*>(a.vp) + base), 0, nbytes, kBufferWord3);
+#pragma unroll
+      for (int i = 0; i < NI / NH; ++i) {
+        const int row = i * RPI + srow;
+        const bool live = pvalid && th + row < t_end && chunk_in_d;
+        const int off =
+            live ? static_cast<int>(((int64_t)(slot0 + row) * a.s_tok + schunk * 8) * sizeof(T))
+                 : -16;
+        sk[half * (NI / NH) + i] = __builtin_amdgcn_raw_buffer_load_b128(rK, off, 0, kLoadNT);
+        sv[half * (NI / NH) + i] = __builtin_amdgcn_raw_buffer_load_b128(rV, off, 0, kLoadNT);
+      }
+      if (pvalid) valid |= P16 ? 1 << half : 3;
     }
-    return pvalid;
+    return valid;
   };
 
-  bool pvalid = issue(t_begin);
+  int pvalid = issue(t_begin);
   issue_bias(t_begin);
   finish_q(qop);
   for (int t = t_begin; t < t_end; t += kStep) {
@@ -367,7 +379,7 @@ __device__ __forceinline__ void rows_range(const DecodeArgs& a, int b, int kvh, 
 #pragma unroll
         for (int i = 0; i < 4; ++i) bcu[gi][i] = bnx[gi][i];
     }
-    const bool cur_valid = pvalid;
+    const int cur_valid = pvalid;
     pvalid = issue(t + kStep);
     if (t + kStep < t_end) issue_bias(t + kStep);
     lc_compiler_fence();
@@ -387,7 +399,8 @@ __device__ __forceinline__ void rows_range(const DecodeArgs& a, int b, int kvh, 
     for (int gi = 0; gi < 2; ++gi)
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
-        const bool live = cur_valid && t + gi * 16 + q4 * 4 + i < t_end;
+        const bool live =
+            (P16 ? (cur_valid >> gi) & 1 : cur_valid != 0) && t + gi * 16 + q4 * 4 + i < t_end;
         const float x = HB ? fmaf(sacc[gi][i], a.scale_log2, bcu[gi][i])
                            : sacc[gi][i] * a.scale_log2;
         sc[gi][i] = live ? x : -INFINITY;
@@ -668,7 +681,7 @@ __device__ __forceinline__ int ordered_pair(const DecodeArgs& a, const int (&li)
 // live ranks is handed out in the order the workgroups start, so the faster
 // XCDs take more of the short final splits (which workgroup computes a split
 // changes nothing in its partials).
-template <typename T, int DPAD, bool HB, bool STEP, bool PRE, bool ORD = false>
+template <typename T, int DPAD, bool HB, bool STEP, bool PRE, bool ORD = false, bool P16 = false>
 __global__ __launch_bounds__(64 * cluster_waves<DPAD>()) void paged_decode_cluster_kernel(
     DecodeArgs a, T* __restrict__ out, int64_t o_sb, int64_t o_sh, float* __restrict__ lse_out,
     StepArgs sa) {
@@ -856,7 +869,7 @@ __global__ __launch_bounds__(64 * cluster_waves<DPAD>()) void paged_decode_clust
           },
           my_k, my_v, o, m_ref, l_lane, row_entry, window_base);
     } else {
-      rows_range<T, DPAD, HB, PRE>(
+      rows_range<T, DPAD, HB, PRE, P16>(
           a, b, kvh, h, head_ok, t_begin, t_end,
           [&](v8 (&qop)[KS]) { load_q<T, DPAD>(a, b, h, kvh * a.G, head_ok, q4, qop); },
           [](v8 (&)[KS]) {}, my_k, my_v, o, m_ref, l_lane, row_entry, window_base);
@@ -1275,7 +1288,10 @@ int launch_cluster(const DecodeArgs& a, void* out, int64_t o_sb, int64_t o_sh, f
       n_wg > lc_cu_count() &&
       n_wg * threads < (1LL << 32)) {  // a 1-D dispatch's work-items fit 32 bits
     const dim3 g1(static_cast<unsigned>(n_wg));
-    if (a.bias != nullptr && pre)
+    if (a.P % kStep != 0)
+      paged_decode_cluster_kernel<T, DPAD, false, false, false, true, true>
+          <<<g1, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
+    else if (a.bias != nullptr && pre)
       paged_decode_cluster_kernel<T, DPAD, true, false, true, true>
           <<<g1, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
     else if (a.bias != nullptr)
@@ -1287,7 +1303,10 @@ int launch_cluster(const DecodeArgs& a, void* out, int64_t o_sb, int64_t o_sh, f
     else
       paged_decode_cluster_kernel<T, DPAD, false, false, false, true>
           <<<g1, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
-  } else if (a.bias != nullptr && pre)
+  } else if (a.P % kStep != 0)
+    paged_decode_cluster_kernel<T, DPAD, false, false, false, false, true>
+        <<<grid, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
+  else if (a.bias != nullptr && pre)
     paged_decode_cluster_kernel<T, DPAD, true, false, true>
         <<<grid, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
   else if (a.bias != nullptr)
@@ -1471,7 +1490,12 @@ int paged_decode_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh
   const int64_t span = max_splits == 1 ? max_pages_per_seq * page_size : split_tokens;
   const int64_t wave_tokens = ((span + kStep - 1) / kStep + waves - 1) / waves * kStep;
   const int64_t units = B * Hkv * ((Hq / Hkv + 15) / 16);
-  const bool cluster = row_pages &&
+  // Pages of 16 tokens run the workgroup splits too, unmasked, two
+  // page lookups a step: 34 us against 62 us for one wave per split with a
+  // page lookup per lane (16 sequences of up to 4000 tokens, cold).
+  const bool half_pages = page_size == kStep / 2 && a.bias == nullptr &&
+                          ((page_size - 1) * kv_s_tok + D) * esz < (1LL << 31);
+  const bool cluster = (row_pages || half_pages) &&
                        (max_splits == 1 || split_tokens >= 2048 || units * max_splits <= 512) &&
                        (wave_tokens - 1) / page_size + 2 <= 64;
   hipStream_t st = lc_stream(stream);

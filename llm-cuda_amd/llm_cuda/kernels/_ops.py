@@ -811,20 +811,22 @@ def single_split_fits(capacity_tokens: int, page_size: int, head_dim: int) -> bo
 def takes_workgroup_splits(units: int, split_tokens: int, max_splits: int, page_size: int,
                            head_dim: int, capacity_tokens: int) -> bool:
     """The library's choice between one workgroup per split and one wave per
-    split (mirrors lc_paged_decode_fwd): workgroups for a single split, splits
-    of >= 2048 tokens, or grids of <= 512 splits."""
+    split (mirrors lc_paged_decode_fwd for unmasked calls): workgroups for a
+    single split, splits of >= 2048 tokens, or grids of <= 512 splits, on pages
+    of 16 or a multiple of 32 tokens."""
     span = capacity_tokens if max_splits == 1 else split_tokens
-    return (page_size % 32 == 0 and _wave_window_fits(span, page_size, head_dim)
+    return ((page_size % 32 == 0 or page_size == 16) and _wave_window_fits(span, page_size, head_dim)
             and (max_splits == 1 or split_tokens >= 2048 or units * max_splits <= 512))
 
 
 def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens: int,
                         page_size: int = 64, head_dim: int = 128,
-                        uniform_length: int | None = None, n_cus: int = 256) -> int:
+                        uniform_length: int | None = None, n_cus: int = 256,
+                        masked: bool = False) -> int:
     """Tokens per split.
 
     units = batch x kv heads x groups of <= 16 query heads. Where the page
-    size allows workgroup splits (a multiple of 32 tokens):
+    size allows workgroup splits (a multiple of 32 tokens, or 16 without a mask):
       * uniform_length given (every sequence holds that many tokens, as in a
         batched decode step): the fewest splits per unit s whose units * s
         fill whole rounds of the CUs to >= 90%, each split a 1/s share of the
@@ -844,20 +846,26 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
         2's shape); one round of the CUs for fewer units, whatever the batch
         (16 sequences of 1-16K tokens, 128 units: 115.7 us at 8192 against
         127-133 us at 512-2048).
-    Where the library would run such a split size with one wave per split
-    instead (see takes_workgroup_splits), or pages are not a multiple of 32,
-    one-wave splits: 512 tokens, shrunk until there are >= 1024 of them.
+    On pages of 16 tokens each rule takes more splits where a wave's share
+    would touch over 64 pages. Where the library would run such a split size
+    with one wave per split instead (see takes_workgroup_splits), or on other
+    page sizes, one-wave splits: 512 tokens, shrunk until there are >= 1024 of them.
     """
     units = batch * n_kv_heads * ((group + 15) // 16)
     if units == 0:  # an empty batch launches nothing; any valid split will do
         return max(64, -(-capacity_tokens // 64) * 64)
-    if page_size % 32 == 0 and capacity_tokens > 0:
+    half_pages = page_size == 16 and not masked
+    if (page_size % 32 == 0 or half_pages) and capacity_tokens > 0:
+        def fits(s: int) -> bool:  # (pages of 32 tokens up: as ever, checked at the end)
+            return not half_pages or _wave_window_fits(
+                -(-(-(-capacity_tokens // s)) // 64) * 64, page_size, head_dim)
+
         if uniform_length is not None:
             length = max(1, min(int(uniform_length), capacity_tokens))
             s = 1
             while s < 64:
                 n = units * s
-                if n >= n_cus and n / (n_cus * -(-n // n_cus)) >= 0.9:
+                if n >= n_cus and n / (n_cus * -(-n // n_cus)) >= 0.9 and fits(s):
                     break
                 s += 1
             split = -(-(-(-length // s)) // 64) * 64
@@ -870,9 +878,13 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
                 s += 1
         elif units >= n_cus:
             s = -(-8 * n_cus // units)
+            while s < 64 and not fits(s):
+                s += 1
             split = -(-(-(-capacity_tokens // s)) // 64) * 64
         else:
             s = max(1, n_cus // units)
+            while s < 64 and not fits(s):
+                s += 1
             split = -(-(-(-capacity_tokens // s)) // 64) * 64
         if s == 1 or split >= capacity_tokens:
             split = -(-capacity_tokens // 64) * 64
@@ -956,7 +968,7 @@ def _paged_decode(q: torch.Tensor, key_pages: torch.Tensor, value_pages: torch.T
     G = Hq // Hkv
     if split_tokens is None:
         split_tokens = choose_split_tokens(B, Hkv, G, capacity, P, D, uniform_length,
-                                           _cu_count(dev))
+                                           _cu_count(dev), attention_mask is not None)
     max_splits = max(1, (capacity + split_tokens - 1) // split_tokens)
     if scale is None:
         scale = 1.0 / math.sqrt(D)
