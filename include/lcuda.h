@@ -171,6 +171,14 @@ LC_API int lc_prefill_attn_fwd_ws(const void* q, const void* k, const void* v, v
  * (delta = rowsum(dO*O), and lse * log2(e)). */
 LC_API int64_t lc_prefill_attn_bwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq);
 
+/* Bytes of workspace an unmasked bf16/f16 lc_prefill_attn_bwd can use past
+ * those, for fp32 sums of key blocks that several workgroups share (short or
+ * few sequences, whose first key block would otherwise end long after the
+ * rest); without them every key block is one workgroup's. 0: no use for any. */
+LC_API int64_t lc_prefill_attn_bwd_split_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                               int64_t Skv, int64_t D, int64_t q_offset,
+                                               int has_bias, int dtype);
+
 /* Causal attention backward with native GQA: given the forward's o and lse
  * (lc_prefill_attn_fwd) and the output gradient dout, writes
  *   dq[b,h,i]   = scale * sum_j dS_ij k[b,h/G,j]

@@ -58,6 +58,11 @@ struct BwdArgs {
   int64_t bs[4];
   int bias_dtype;
   int bias_vec;
+  // dK/dV key blocks shared by several workgroups (the SPLIT instances): a
+  // block's tiles are dealt out in shares of at most dkv_share, and the shares
+  // of the blocks that have more than one leave fp32 sums in dkv_part.
+  float* dkv_part;
+  int dkv_share;
 };
 
 // ---------------------------------------------------------------------------
@@ -940,7 +945,23 @@ attn_bwd_dq_mfma_kernel(BwdArgs a, int hw, int n_rbg) {
 // so a lane's bias values (one key, 32 query rows) are read one element each;
 // bias tiles keep the plain phase order (the 32 bias registers do not fit the
 // pipeline's budget).
-template <typename T, int DPAD, int BIAS>
+// Tiles of a key block: the (query tile, head of the group) pairs that see any
+// of its keys. Never more for a later block.
+__device__ __host__ __forceinline__ int dkv_tiles(int kb, int n_qt, int q_offset, int G) {
+  const int first = kb * kBkKeys - q_offset;
+  const int nq = n_qt - (first > 0 ? first : 0) / kBwTile;
+  return nq > 0 ? nq * G : 0;
+}
+__device__ __host__ __forceinline__ int dkv_shares(int tiles, int share) {
+  return tiles <= share ? 1 : (tiles + share - 1) / share;
+}
+
+// SPLIT: a causal grid of few key blocks ends with its first block, whose tiles
+// are twice the mean, and a short one leaves most CUs without a block: the
+// blocks' tiles are dealt out in shares instead (workgroup i: share item
+// i / units, the blocks' shares in turn; unit i mod units). Shares of blocks
+// that have several write fp32 sums, added in share order by dkv_reduce_kernel.
+template <typename T, int DPAD, int BIAS, bool SPLIT = false>
 __global__ __launch_bounds__(64 * kBkWaves) __attribute__((amdgpu_waves_per_eu(1, 1))) void
 attn_bwd_dkv_mfma_kernel(BwdArgs a) {
   typedef Mfma32<T> Ops;
@@ -966,8 +987,27 @@ attn_bwd_dkv_mfma_kernel(BwdArgs a) {
   const int l32 = lane & 31;
   const int hh = lane >> 5;
   const int n_units = a.B * a.Hkv;
-  const int kb = blockIdx.x / n_units;
+  int kb = blockIdx.x / n_units;
   const int unit = blockIdx.x - kb * n_units;
+  int share = 0, shares = 1;
+  if constexpr (SPLIT) {
+    int item = kb;
+    const int n_qt_s = (a.Sq + kBwTile - 1) / kBwTile;
+    kb = 0;
+    shares = dkv_shares(dkv_tiles(0, n_qt_s, a.q_offset, a.G), a.dkv_share);
+    while (item >= shares) {
+      item -= shares;
+      ++kb;
+      shares = dkv_shares(dkv_tiles(kb, n_qt_s, a.q_offset, a.G), a.dkv_share);
+    }
+    share = item;
+    // (opaque, as the block id's quotient is: the tile loop must not see the
+    // path they came by)
+    kb = __builtin_amdgcn_readfirstlane(kb);
+    share = __builtin_amdgcn_readfirstlane(share);
+    shares = __builtin_amdgcn_readfirstlane(shares);
+    asm volatile("" : "+s"(kb), "+s"(share), "+s"(shares));
+  }
   const int kvh = unit % a.Hkv;
   const int b = unit / a.Hkv;
   // This wave's first key. The pipelined path needs it wave-uniform (scalar
@@ -1234,6 +1274,12 @@ attn_bwd_dkv_mfma_kernel(BwdArgs a) {
     }
   };
 
+  // This workgroup's iterations (a share starts on an even one: buffer 0).
+  int it0 = 0, it1 = n_iter;
+  if constexpr (SPLIT) {
+    it0 = static_cast<int>((int64_t)n_iter * share / shares) & ~1;
+    it1 = share + 1 == shares ? n_iter : static_cast<int>((int64_t)n_iter * (share + 1) / shares) & ~1;
+  }
   // MASK: false / true for tiles known to be unmasked / on the diagonal,
   // kRuntimeMask to pick per tile (the bias path).
   auto iteration = [&](int it, auto par_c, auto mask_c) __attribute__((always_inline)) {
@@ -1249,7 +1295,7 @@ attn_bwd_dkv_mfma_kernel(BwdArgs a) {
           tile(qt, par_c, std::true_type{});
       }
     } else {
-      if (it + 1 < n_iter) fetch(it + 1, other);
+      if (it + 1 < it1) fetch(it + 1, other);
       tile(qt, par_c, mask_c);
     }
     pf_barrier<true>();
@@ -1268,7 +1314,7 @@ attn_bwd_dkv_mfma_kernel(BwdArgs a) {
     if (it < end) iteration(it, std::integral_constant<int, 0>{}, mask_c);
   };
 
-  if (n_iter > 0) fetch(0, std::integral_constant<int, 0>{});
+  if (it0 < it1) fetch(it0, std::integral_constant<int, 0>{});
   pf_barrier<true>();
   if constexpr (BIAS != 0) {
     run(0, n_iter, std::integral_constant<int, kRuntimeMask>{});
@@ -1276,17 +1322,108 @@ attn_bwd_dkv_mfma_kernel(BwdArgs a) {
     // Waves whose keys all lie past Skv run the tiles on zero K/V operands and
     // store nothing; every wave passes the same barriers.
     const int n_nomask = min(n_iter, max(0, n_qt - qt_nomask) * a.G);
-    run(0, n_nomask, std::false_type{});
-    run(n_nomask, n_iter, std::true_type{});
+    run(it0, min(n_nomask, it1), std::false_type{});
+    run(max(it0, n_nomask), it1, std::true_type{});
   }
 
   if (!key_ok) return;
+  if constexpr (SPLIT) {
+    if (shares > 1) {
+      // (blocks with several shares come first, so the block id counts them)
+      float* p = a.dkv_part + (int64_t)blockIdx.x * (2 * kBkKeys * DPAD) +
+                 (int64_t)(wave_s * 32 + l32) * DPAD;
+      store_transposed<float, DTL>(p, dk, 1.0f, hh, DPAD);
+      store_transposed<float, DTL>(p + kBkKeys * DPAD, dv, 1.0f, hh, DPAD);
+      return;
+    }
+  }
   store_transposed<T, DTL>(static_cast<T*>(a.dk) + b * a.dks[0] + (int64_t)kvh * a.dks[1] +
                                (int64_t)kj * a.dks[2],
                            dk, a.scale, hh, a.D);
   store_transposed<T, DTL>(static_cast<T*>(a.dv) + b * a.dvs[0] + (int64_t)kvh * a.dvs[1] +
                                (int64_t)kj * a.dvs[2],
                            dv, 1.0f, hh, a.D);
+}
+
+// Adds the shares' sums of the key blocks that have several: one workgroup per
+// 32 keys of a (block, unit), 16 bytes of dK and dV per thread and share. Bound
+// by reading the sums once.
+template <typename T, int DPAD>
+__global__ __launch_bounds__(256) void dkv_reduce_kernel(BwdArgs a) {
+  typedef T t4 __attribute__((ext_vector_type(4)));
+  const int n_units = a.B * a.Hkv;
+  const int n_qt = (a.Sq + kBwTile - 1) / kBwTile;
+  const int part = blockIdx.x & (kBkKeys / 32 - 1);
+  const int kb = (blockIdx.x / (kBkKeys / 32)) / n_units;
+  const int unit = (blockIdx.x / (kBkKeys / 32)) - kb * n_units;
+  int first = 0;  // the block's first share item
+  for (int i = 0; i < kb; ++i)
+    first += dkv_shares(dkv_tiles(i, n_qt, a.q_offset, a.G), a.dkv_share);
+  const int shares = dkv_shares(dkv_tiles(kb, n_qt, a.q_offset, a.G), a.dkv_share);
+  const int kvh = unit % a.Hkv, b = unit / a.Hkv;
+  for (int e = threadIdx.x; e < 32 * (DPAD / 4); e += 256) {
+    const int row = part * 32 + e / (DPAD / 4), d = (e % (DPAD / 4)) * 4;
+    const int kj = kb * kBkKeys + row;
+    if (kj >= a.Skv || d >= a.D) continue;
+    f32x4_t dk = {0.f, 0.f, 0.f, 0.f}, dv = dk;
+    for (int s = 0; s < shares; ++s) {
+      const float* p = a.dkv_part + ((int64_t)(first + s) * n_units + unit) * (2 * kBkKeys * DPAD) +
+                       row * DPAD + d;
+      dk += *reinterpret_cast<const f32x4_t*>(p);
+      dv += *reinterpret_cast<const f32x4_t*>(p + kBkKeys * DPAD);
+    }
+    t4 wk, wv;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      wk[i] = lc_from_f32<T>(dk[i] * a.scale);
+      wv[i] = lc_from_f32<T>(dv[i]);
+    }
+    *reinterpret_cast<t4*>(static_cast<T*>(a.dk) + b * a.dks[0] + (int64_t)kvh * a.dks[1] +
+                           (int64_t)kj * a.dks[2] + d) = wk;
+    *reinterpret_cast<t4*>(static_cast<T*>(a.dv) + b * a.dvs[0] + (int64_t)kvh * a.dvs[1] +
+                           (int64_t)kj * a.dvs[2] + d) = wv;
+  }
+}
+
+// How an unmasked MFMA call's dK/dV grid is dealt out (share 0: one workgroup
+// per key block). A workgroup has a CU to itself, so a grid takes as long as its
+// first block unless the blocks fill several rounds: where that block has over
+// 1.4 times a CU's mean share of all tiles, blocks are dealt out in shares of 1.3
+// times the mean (at the mean itself a second round of small shares starts; the
+// fp32 sums and their launch cost more at smaller ones). us a backward, whole
+// blocks / 1.0 / 1.3 / 1.6 of the mean, D 128, 32/8 heads: [1, 512] 85 / 57 /
+// 57 / 56, [1, 1024] 152 / 100 / 82 / 83, [1, 2048] 295 / 208 / 172 / 181,
+// [2, 2048] 337 / 315 / 294 / 308.
+struct DkvPlan {
+  int share;     // tiles per share
+  int items;     // share items of a unit
+  int multi;     // of those, the items of blocks with several shares
+  int blocks;    // blocks with several shares
+};
+constexpr int kDkvMinShare = 4;
+DkvPlan dkv_plan(int64_t units, int64_t Sq, int64_t Skv, int64_t q_offset, int G) {
+  const int n_qt = static_cast<int>((Sq + kBwTile - 1) / kBwTile);
+  const int n_kb = static_cast<int>((Skv + kBkKeys - 1) / kBkKeys);
+  int64_t total = 0;
+  for (int kb = 0; kb < n_kb; ++kb) total += dkv_tiles(kb, n_qt, (int)q_offset, G);
+  const int64_t mean = (total * units + lc_cu_count() - 1) / lc_cu_count();
+  DkvPlan p{0, 0, 0, 0};
+  const int most = n_kb > 0 ? dkv_tiles(0, n_qt, (int)q_offset, G) : 0;
+  const int64_t share = (mean * 13 + 9) / 10;
+  if (most <= 2 * kDkvMinShare || most * 5 <= mean * 7) return p;
+  p.share = static_cast<int>(share > kDkvMinShare ? share : kDkvMinShare);
+  for (int kb = 0; kb < n_kb; ++kb) {
+    const int s = dkv_shares(dkv_tiles(kb, n_qt, (int)q_offset, G), p.share);
+    p.items += s;
+    if (s > 1) {
+      p.multi += s;
+      ++p.blocks;
+    }
+  }
+  return p;
+}
+int64_t dkv_part_bytes(const DkvPlan& p, int64_t units, int64_t D) {
+  return p.share == 0 ? 0 : units * p.multi * (2LL * kBkKeys * (D <= 64 ? 64 : 128) * 4);
 }
 
 static int gcd_int(int x, int y) {
@@ -1314,8 +1451,15 @@ void launch_dkv_mfma(const BwdArgs& a, unsigned nwg, hipStream_t st) {
     attn_bwd_dkv_mfma_kernel<T, 128, BIAS><<<nwg, 64 * kBkWaves, 0, st>>>(a);
 }
 
+template <typename T, int DPAD>
+void launch_dkv_split(const BwdArgs& a, const DkvPlan& p, int units, hipStream_t st) {
+  attn_bwd_dkv_mfma_kernel<T, DPAD, 0, true>
+      <<<(unsigned)(p.items * units), 64 * kBkWaves, 0, st>>>(a);
+  dkv_reduce_kernel<T, DPAD><<<(unsigned)(p.blocks * units * (kBkKeys / 32)), 256, 0, st>>>(a);
+}
+
 template <typename T>
-int launch_bwd_mfma(const BwdArgs& a, hipStream_t st) {
+int launch_bwd_mfma(BwdArgs a, int64_t part_bytes, hipStream_t st) {
   const int hw = gcd_int(a.G, kBwWaves);
   const int rbw = kBwWaves / hw;
   const int n_rb = (a.Sq + kBwRows - 1) / kBwRows;
@@ -1333,7 +1477,21 @@ int launch_bwd_mfma(const BwdArgs& a, hipStream_t st) {
     else
       launch_dq_mfma<T, 2>(a, (unsigned)nwg_q, hw, n_rbg, st);
   }
-  if (nwg_k > 0) {
+  const int units = a.B * a.Hkv;
+  DkvPlan plan{0, 0, 0, 0};
+  if (bias == 0 && part_bytes > 0 && nwg_k > 0) {
+    plan = dkv_plan(units, a.Sq, a.Skv, a.q_offset, a.G);
+    if (dkv_part_bytes(plan, units, a.D) > part_bytes ||
+        (int64_t)plan.items * units * (kBkKeys / 32) >= (1LL << 31))
+      plan.share = 0;
+  }
+  if (plan.share > 0) {
+    a.dkv_share = plan.share;
+    if (a.D <= 64)
+      launch_dkv_split<T, 64>(a, plan, units, st);
+    else
+      launch_dkv_split<T, 128>(a, plan, units, st);
+  } else if (nwg_k > 0) {
     if (bias == 0)
       launch_dkv_mfma<T, 0>(a, (unsigned)nwg_k, st);
     else if (bias == 1)
@@ -1363,7 +1521,7 @@ int launch_delta(const void* o, const int64_t* o_strides, const BwdArgs& a, floa
 
 template <typename T>
 int run_bwd(const void* o, const int64_t* o_strides, BwdArgs a, float* delta, float* lse2,
-            bool mfma, hipStream_t st) {
+            int64_t part_bytes, bool mfma, hipStream_t st) {
   a.delta = delta;
   a.lse2 = lse2;
   a.o = o;
@@ -1371,7 +1529,7 @@ int run_bwd(const void* o, const int64_t* o_strides, BwdArgs a, float* delta, fl
   if constexpr (!std::is_same<T, float>::value) {
     // The dQ kernel forms delta and lse2 for every query row (an empty query
     // side needs neither).
-    if (mfma) return launch_bwd_mfma<T>(a, st);
+    if (mfma) return launch_bwd_mfma<T>(a, part_bytes, st);
   }
   int rc = launch_delta<T>(o, o_strides, a, delta, lse2, st);
   if (rc != LC_OK) return rc;
@@ -1388,6 +1546,16 @@ extern "C" {
 int64_t lc_prefill_attn_bwd_workspace_bytes(int64_t B, int64_t Hq, int64_t Sq) {
   if (B < 0 || Hq < 0 || Sq < 0) return -1;
   return 2 * (((B * Hq * Sq * 4) + 255) / 256 * 256);
+}
+
+int64_t lc_prefill_attn_bwd_split_bytes(int64_t B, int64_t Hq, int64_t Hkv, int64_t Sq,
+                                        int64_t Skv, int64_t D, int64_t q_offset, int has_bias,
+                                        int dtype) {
+  if (B <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv != 0 || Sq <= 0 || Skv <= 0 || D <= 0 ||
+      Sq >= (1LL << 31) || Skv >= (1LL << 31) || q_offset < 0 || q_offset >= (1LL << 30) ||
+      has_bias || dtype == LC_DTYPE_F32 || D % 8 != 0 || D > 128)
+    return 0;
+  return dkv_part_bytes(dkv_plan(B * Hkv, Sq, Skv, q_offset, (int)(Hq / Hkv)), B * Hkv, D);
 }
 
 int lc_prefill_attn_bwd(const void* q, const void* k, const void* v, const void* o,
@@ -1467,6 +1635,8 @@ int lc_prefill_attn_bwd(const void* q, const void* k, const void* v, const void*
     for (int i = 0; i < 4; ++i) a.bs[i] = bias_strides[i];
   float* delta = static_cast<float*>(workspace);
   float* lse2 = delta + need / 8;
+  a.dkv_part = delta + need / 4;  // what the caller gave past the two row arrays
+  const int64_t part_bytes = workspace_bytes - need;
   const int64_t esz = lc_dtype_size(dtype);
   bool mfma = (dtype == LC_DTYPE_BF16 || dtype == LC_DTYPE_F16) && D % 8 == 0 && D <= 128;
   for (const void* p : {q, k, v, o, dout, (const void*)dq, (const void*)dk, (const void*)dv}) mfma = mfma && lc_aligned(p, 16);
@@ -1505,11 +1675,11 @@ int lc_prefill_attn_bwd(const void* q, const void* k, const void* v, const void*
   hipStream_t st = lc_stream(stream);
   switch (dtype) {
     case LC_DTYPE_F32:
-      return run_bwd<float>(o, o_strides, a, delta, lse2, f32, st);
+      return run_bwd<float>(o, o_strides, a, delta, lse2, 0, f32, st);
     case LC_DTYPE_BF16:
-      return run_bwd<bf16_t>(o, o_strides, a, delta, lse2, mfma, st);
+      return run_bwd<bf16_t>(o, o_strides, a, delta, lse2, part_bytes, mfma, st);
     case LC_DTYPE_F16:
-      return run_bwd<f16_t>(o, o_strides, a, delta, lse2, mfma, st);
+      return run_bwd<f16_t>(o, o_strides, a, delta, lse2, part_bytes, mfma, st);
     default:
       return lc_fail(LC_EINVAL, "lc_prefill_attn_bwd: unknown dtype %d", dtype);
   }

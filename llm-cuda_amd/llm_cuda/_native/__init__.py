@@ -71,6 +71,10 @@ _SIGNATURES = {
          ctypes.c_float, ctypes.c_int, _c_p],
     ),
     "lc_prefill_attn_bwd_workspace_bytes": (_c_i64, [_c_i64, _c_i64, _c_i64]),
+    "lc_prefill_attn_bwd_split_bytes": (
+        _c_i64,
+        [_c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, _c_i64, ctypes.c_int, ctypes.c_int],
+    ),
     "lc_prefill_attn_bwd": (
         ctypes.c_int,
         [_c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_p, _c_i64, _c_i64, _c_i64, _c_i64,

@@ -450,6 +450,8 @@ def prefill_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     dv = torch.empty((B, Hkv, Skv, D), dtype=q.dtype, device=dev)
     lib = nat.load()
     ws_bytes = lib.lc_prefill_attn_bwd_workspace_bytes(B, Hq, Sq)
+    ws_bytes += lib.lc_prefill_attn_bwd_split_bytes(B, Hq, Hkv, Sq, Skv, D, int(q_offset),
+                                                    int(bias is not None), nat.lc_dtype(q))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
     with _DeviceGuard(dev):
         rc = lib.lc_prefill_attn_bwd(
