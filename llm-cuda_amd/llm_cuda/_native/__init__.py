@@ -9,6 +9,7 @@ there is no silent fallback to another implementation.
 from __future__ import annotations
 
 import ctypes
+import functools
 import threading
 from pathlib import Path
 
@@ -219,6 +220,22 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
     The HIP kernels are the only implementation of the attention path: host
     (CPU) tensors are rejected instead of being computed another way.
     """
+    # (Tensor.get_device is the cheapest question; the details only on an error.)
+    first, index = None, -1
+    for t in tensors:
+        if t is None:
+            continue
+        i = t.get_device()
+        if first is None:
+            first, index = t, i
+        if i < 0 or i != index or not t.is_cuda:
+            _refuse_devices(tensors)
+    if first is None:
+        raise RuntimeError("no tensor given")
+    return first.device
+
+
+def _refuse_devices(tensors) -> None:
     dev = None
     for t in tensors:
         if t is None:
@@ -232,13 +249,21 @@ def require_device(*tensors: torch.Tensor) -> torch.device:
             dev = t.device
         elif t.device != dev:
             raise RuntimeError(f"tensors on different devices: {dev} and {t.device}")
-    if dev is None:
-        raise RuntimeError("no tensor given")
-    return dev
 
 
 def stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The handle of torch's current stream of the device (what
+    torch.cuda.current_stream(device).cuda_stream gives, without its objects)."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
+
+
+@functools.lru_cache(maxsize=4096)
+def size(name: str, *args: int) -> int:
+    """An entry point that maps sizes to a size (workspace bytes, counts): a
+    pure function of its integers, called once for each."""
+    return getattr(load(), name)(*args)
 
 
 def strides4(t: torch.Tensor):

@@ -8,6 +8,8 @@ device tensors; anything else raises (there is no second implementation).
 from __future__ import annotations
 
 import contextlib
+import ctypes
+import functools
 import math
 
 import torch
@@ -17,10 +19,11 @@ from torch.nn.modules import module as _module
 from llm_cuda import _native as nat
 
 
-def _i64arr(vals):
-    import ctypes
+_I64X = {n: ctypes.c_int64 * n for n in range(1, 6)}
 
-    return (ctypes.c_int64 * len(vals))(*vals)
+
+def _i64arr(vals):
+    return _I64X[len(vals)](*vals)
 
 
 def _stream(dev: torch.device) -> int:
@@ -60,6 +63,14 @@ class _DeviceGuard:
         return False
 
 
+_HERE = contextlib.nullcontext()
+
+
+def _guard(dev: torch.device):
+    """A context in which `dev` is current: nothing to do where it already is."""
+    return _HERE if torch._C._cuda_getDevice() == dev.index else _DeviceGuard(dev)
+
+
 # ---------------------------------------------------------------------------
 # Forward-only kernels under autograd
 # ---------------------------------------------------------------------------
@@ -81,8 +92,22 @@ class _ForwardOnly(torch.autograd.Function):
 
 
 def _records_grad(*tensors) -> bool:
-    return torch.is_grad_enabled() and any(
-        t is not None and t.requires_grad for t in tensors)
+    if torch.is_grad_enabled():
+        for t in tensors:
+            if t is not None and t.requires_grad:
+                return True
+    return False
+
+
+def _rows(x: torch.Tensor, cols: int):
+    """x's rows of `cols` elements: (tensor, row stride) with unit stride inside
+    a row. A contiguous x is taken as it stands, without a view."""
+    if x.is_contiguous() and cols > 0:
+        return x, cols
+    x2 = x.reshape(-1, cols)
+    if x2.stride(-1) != 1:
+        x2 = x2.contiguous()
+    return x2, x2.stride(0)
 
 
 # ---------------------------------------------------------------------------
@@ -100,20 +125,18 @@ def _rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor
     if weight.dim() != 1 or weight.shape[0] != x.shape[-1]:
         raise ValueError(f"weight shape {tuple(weight.shape)} does not match hidden {x.shape[-1]}")
     hidden = x.shape[-1]
-    x2 = x.reshape(-1, hidden)
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
+    x2, xs = _rows(x, hidden)
     w = weight if weight.is_contiguous() else weight.contiguous()
     if w.dtype != x.dtype and w.dtype != torch.float32:
         w = w.to(x.dtype)
-    y = torch.empty((x2.shape[0], hidden), dtype=x.dtype, device=dev)
+    y = torch.empty(x.shape, dtype=x.dtype, device=dev)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_rmsnorm_fwd(
-            x2.data_ptr(), w.data_ptr(), y.data_ptr(), x2.shape[0], hidden, x2.stride(0),
-            y.stride(0), float(eps), nat.lc_dtype(x), nat.lc_dtype(w), _stream(dev))
+            x2.data_ptr(), w.data_ptr(), y.data_ptr(), x.numel() // hidden if hidden else 0, hidden,
+            xs, hidden, float(eps), nat.lc_dtype(x), nat.lc_dtype(w), _stream(dev))
     nat.check(rc, "lc_rmsnorm_fwd")
-    return y.view(x.shape)
+    return y
 
 
 def add_rms_norm(x: torch.Tensor, residual, weight: torch.Tensor, eps: float,
@@ -148,27 +171,23 @@ def _add_rms_norm(x: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
     if weight.dim() != 1 or weight.shape[0] != x.shape[-1]:
         raise ValueError(f"weight shape {tuple(weight.shape)} does not match hidden {x.shape[-1]}")
     hidden = x.shape[-1]
-    x2 = x.reshape(-1, hidden)
-    r2 = residual.reshape(-1, hidden)
-    if inplace and (x2.data_ptr() != x.data_ptr() or x2.stride(-1) != 1):
+    x2, xs = _rows(x, hidden)
+    r2, rs = _rows(residual, hidden)
+    if inplace and x2.data_ptr() != x.data_ptr():
         raise ValueError("inplace add_rms_norm needs x with unit stride over hidden")
-    if x2.stride(-1) != 1:
-        x2 = x2.contiguous()
-    if r2.stride(-1) != 1:
-        r2 = r2.contiguous()
     w = weight if weight.is_contiguous() else weight.contiguous()
     if w.dtype != x.dtype and w.dtype != torch.float32:
         w = w.to(x.dtype)
-    y = torch.empty((x2.shape[0], hidden), dtype=x.dtype, device=dev)
-    s2 = x2 if inplace else torch.empty((x2.shape[0], hidden), dtype=x.dtype, device=dev)
+    y = torch.empty(x.shape, dtype=x.dtype, device=dev)
+    s, ss = (x2, xs) if inplace else (torch.empty(x.shape, dtype=x.dtype, device=dev), hidden)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_add_rmsnorm_fwd(
-            x2.data_ptr(), r2.data_ptr(), w.data_ptr(), y.data_ptr(), s2.data_ptr(), x2.shape[0],
-            hidden, x2.stride(0), r2.stride(0), y.stride(0), s2.stride(0), float(eps),
+            x2.data_ptr(), r2.data_ptr(), w.data_ptr(), y.data_ptr(), s.data_ptr(),
+            x.numel() // hidden if hidden else 0, hidden, xs, rs, hidden, ss, float(eps),
             nat.lc_dtype(x), nat.lc_dtype(w), _stream(dev))
     nat.check(rc, "lc_add_rmsnorm_fwd")
-    return y.view(x.shape), (x if inplace else s2.view(x.shape))
+    return y, (x if inplace else s)
 
 
 def _add_rms_norm_partials(x: torch.Tensor, residual: "PartialSum", weight: torch.Tensor,
@@ -196,7 +215,7 @@ def _add_rms_norm_partials(x: torch.Tensor, residual: "PartialSum", weight: torc
     y = torch.empty((x2.shape[0], hidden), dtype=x.dtype, device=dev)
     s2 = x2 if inplace else torch.empty((x2.shape[0], hidden), dtype=x.dtype, device=dev)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_add_rmsnorm_partials_fwd(
             x2.data_ptr(), parts.data_ptr(), parts.shape[0], parts.stride(0), w.data_ptr(),
             y.data_ptr(), s2.data_ptr(), x2.shape[0], hidden, x2.stride(0), parts.stride(1),
@@ -232,7 +251,7 @@ def _swiglu(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
         u2 = u2.contiguous()
     out = torch.empty((g2.shape[0], cols), dtype=gate.dtype, device=dev)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_swiglu_fwd(
             g2.data_ptr(), u2.data_ptr(), out.data_ptr(), g2.shape[0], cols, g2.stride(0),
             u2.stride(0), out.stride(0), nat.lc_dtype(gate), _stream(dev))
@@ -289,7 +308,7 @@ def _rope(x1: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor,
     o1 = torch.empty((B, H1, S, D), dtype=x1.dtype, device=dev)
     o2 = None if x2 is None else torch.empty(tuple(x2.shape), dtype=x2.dtype, device=dev)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_rope_fwd(
             x1.data_ptr(), o1.data_ptr(), H1, _i64arr(x1.stride()), _i64arr(o1.stride()),
             None if x2 is None else x2.data_ptr(), None if o2 is None else o2.data_ptr(),
@@ -385,17 +404,17 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, q_offse
     lib = nat.load()
     # The ticket of the kernel's dynamic tail (zero-on-exit); a capture before
     # any eager call runs the static order (no counters).
-    counters = _zeroed_counters("prefill", dev, lib.lc_prefill_attn_counter_count(),
+    counters = _zeroed_counters("prefill", dev, nat.size("lc_prefill_attn_counter_count"),
                                 optional=True)
     # Fp32 partials of a call whose keys are split (the library splits no call
     # of under 32 tiles of 64 visible keys; 0 bytes: it does not split this one).
     ws, ws_bytes = None, 0
     if bias is None and Skv > 1984 and Sq + q_offset > 1984:
-        ws_bytes = lib.lc_prefill_attn_workspace_bytes(B, Hq, Hkv, Sq, Skv, D, int(q_offset), 0,
-                                                       nat.lc_dtype(q))
+        ws_bytes = nat.size("lc_prefill_attn_workspace_bytes", B, Hq, Hkv, Sq, Skv, D,
+                            int(q_offset), 0, nat.lc_dtype(q))
         if ws_bytes > 0:
             ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_prefill_attn_fwd_ws(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(),
             None if lse is None else lse.data_ptr(), B, Hq, Hkv, Sq, Skv, D,
@@ -449,11 +468,11 @@ def prefill_attention_backward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     dk = torch.empty((B, Hkv, Skv, D), dtype=q.dtype, device=dev)
     dv = torch.empty((B, Hkv, Skv, D), dtype=q.dtype, device=dev)
     lib = nat.load()
-    ws_bytes = lib.lc_prefill_attn_bwd_workspace_bytes(B, Hq, Sq)
-    ws_bytes += lib.lc_prefill_attn_bwd_split_bytes(B, Hq, Hkv, Sq, Skv, D, int(q_offset),
-                                                    int(bias is not None), nat.lc_dtype(q))
+    ws_bytes = nat.size("lc_prefill_attn_bwd_workspace_bytes", B, Hq, Sq)
+    ws_bytes += nat.size("lc_prefill_attn_bwd_split_bytes", B, Hq, Hkv, Sq, Skv, D, int(q_offset),
+                         int(bias is not None), nat.lc_dtype(q))
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_prefill_attn_bwd(
             q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), lse.data_ptr(),
             dout.data_ptr(), dq.data_ptr(), dk.data_ptr(), dv.data_ptr(), B, Hq, Hkv, Sq, Skv, D,
@@ -498,10 +517,10 @@ def lm_head_argmax(hidden: torch.Tensor, weight: torch.Tensor, return_max: bool 
     ids = torch.empty(B, dtype=torch.int64, device=dev)
     mx = torch.empty(B, dtype=torch.float32, device=dev) if return_max else None
     lib = nat.load()
-    ws_bytes = lib.lc_lm_head_argmax_workspace_bytes(B, V)
+    ws_bytes = nat.size("lc_lm_head_argmax_workspace_bytes", B, V)
     ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
-    counters = _zeroed_counters("lm_head", dev, lib.lc_lm_head_argmax_counter_count())
-    with _DeviceGuard(dev):
+    counters = _zeroed_counters("lm_head", dev, nat.size("lc_lm_head_argmax_counter_count"))
+    with _guard(dev):
         rc = lib.lc_lm_head_argmax(
             hidden.data_ptr(), hidden.stride(0), weight.data_ptr(), weight.stride(0), B, K, V,
             ids.data_ptr(), None if mx is None else mx.data_ptr(), ws.data_ptr(), ws.numel(),
@@ -535,10 +554,9 @@ def _zeroed_counters(kind: str, dev: torch.device, n: int, optional: bool = Fals
     exists), so replays of graphs holding such calls must not overlap on one
     device. A capture before any eager call raises, or returns None when
     `optional` (for kernels whose counters are an optimisation only)."""
-    capturing = torch.cuda.is_current_stream_capturing()
-    keys = [(kind, dev.type, dev.index, "graphs")]
-    if not capturing:
-        keys.append((kind, dev.type, dev.index, _stream(dev)))
+    capturing = torch._C._cuda_isCurrentStreamCapturing()
+    graphs = (kind, dev.type, dev.index, "graphs")
+    keys = (graphs,) if capturing else (graphs, (kind, dev.type, dev.index, _stream(dev)))
     for key in keys:
         buf = _COUNTERS.get(key)
         if buf is None or buf.numel() < n:
@@ -635,12 +653,12 @@ def decode_linear(x: torch.Tensor, weight: torch.Tensor, swiglu: bool = False,
         return y
     mode = 1 if swiglu else 0
     lib = nat.load()
-    ws_bytes = lib.lc_decode_linear_workspace_bytes(M, N, K, mode, int(splits))
+    ws_bytes = nat.size("lc_decode_linear_workspace_bytes", M, N, K, mode, int(splits))
     if ws_bytes < 0:
         raise ValueError(f"decode_linear: unsupported sizes M={M} N={N} K={K}")
     ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-    counters = _decode_linear_counters(dev, lib.lc_decode_linear_counter_count(N, mode))
-    with _DeviceGuard(dev):
+    counters = _decode_linear_counters(dev, nat.size("lc_decode_linear_counter_count", N, mode))
+    with _guard(dev):
         rc = lib.lc_decode_linear(
             x2.data_ptr(), x2.stride(0), weight.data_ptr(), weight.stride(0), y.data_ptr(), N,
             M, N, K, mode, int(splits), ws.data_ptr(), ws.numel(), counters.data_ptr(),
@@ -700,12 +718,12 @@ def decode_linear_partials(x: torch.Tensor, weight: torch.Tensor, shares: int = 
     weight = weight if weight.stride(-1) == 1 else weight.contiguous()
     M, N = x2.shape[0], weight.shape[0]
     lib = nat.load()
-    S = int(shares) if shares > 0 else lib.lc_decode_linear_partial_count(N, K)
+    S = int(shares) if shares > 0 else nat.size("lc_decode_linear_partial_count", N, K)
     if S < 1:
         raise ValueError(f"decode_linear_partials: unsupported sizes N={N} K={K}")
     parts = torch.empty(S, M, N, dtype=torch.float32, device=dev)
     if M:
-        with _DeviceGuard(dev):
+        with _guard(dev):
             rc = lib.lc_decode_linear_partials(
                 x2.data_ptr(), x2.stride(0), weight.data_ptr(), weight.stride(0),
                 parts.data_ptr(), M, N, K, S, nat.lc_dtype(x), _stream(dev))
@@ -752,18 +770,20 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         raise ValueError(f"x {tuple(x.shape)} and weight {tuple(weight.shape)} do not match")
     dev = nat.require_device(x, weight)
     N, K = weight.shape
-    x2 = x.reshape(-1, K)
-    M = x2.shape[0]
-    if x2.stride(-1) != 1 or (M > 1 and not K <= x2.stride(0) < 2 ** 23):
-        x2 = x2.contiguous()
+    M = x.numel() // K if K else 0
+    x2, xs = _rows(x, K)
+    if M == 1:
+        xs = K
+    elif not K <= xs < 2 ** 23:  # (rows that overlap, or too far apart for the kernel)
+        x2, xs = x2.contiguous(), K
     if weight.stride(-1) != 1 or (N > 1 and weight.stride(0) < K):
         weight = weight.contiguous()
-    y = torch.empty(*x.shape[:-1], N, dtype=torch.float32, device=dev)
+    y = torch.empty((*x.shape[:-1], N), dtype=torch.float32, device=dev)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_linear_f32(
-            x2.data_ptr(), x2.stride(0) if M > 1 else K, weight.data_ptr(),
-            weight.stride(0) if N > 1 else K, y.data_ptr(), N, M, N, K, _stream(dev))
+            x2.data_ptr(), xs, weight.data_ptr(), weight.stride(0) if N > 1 else K, y.data_ptr(),
+            N, M, N, K, _stream(dev))
     nat.check(rc, "lc_linear_f32")
     return y
 
@@ -821,6 +841,7 @@ def takes_workgroup_splits(units: int, split_tokens: int, max_splits: int, page_
             and (max_splits == 1 or split_tokens >= 2048 or units * max_splits <= 512))
 
 
+@functools.lru_cache(maxsize=4096)
 def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens: int,
                         page_size: int = 64, head_dim: int = 128,
                         uniform_length: int | None = None, n_cus: int = 256,
@@ -975,7 +996,7 @@ def _paged_decode(q: torch.Tensor, key_pages: torch.Tensor, value_pages: torch.T
     if scale is None:
         scale = 1.0 / math.sqrt(D)
     lib = nat.load()
-    need = lib.lc_paged_decode_workspace_bytes(B, Hq, D, max_splits)
+    need = nat.size("lc_paged_decode_workspace_bytes", B, Hq, D, max_splits)
     if workspace is None or workspace.numel() * workspace.element_size() < need:
         workspace = torch.empty(max(need, 256), dtype=torch.uint8, device=dev)
     bias = None
@@ -986,9 +1007,9 @@ def _paged_decode(q: torch.Tensor, key_pages: torch.Tensor, value_pages: torch.T
     lse = torch.empty((B, Hq), dtype=torch.float32, device=dev) if return_lse else None
     # The ticket of the longest-first order's dynamic tail (zero-on-exit); a
     # capture before any eager call runs the static order (no counters).
-    counters = _zeroed_counters("paged_decode", dev, lib.lc_paged_decode_counter_count(),
+    counters = _zeroed_counters("paged_decode", dev, nat.size("lc_paged_decode_counter_count"),
                                 optional=True)
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_paged_decode_fwd(
             q4.data_ptr(), q4.stride(0), q4.stride(1), key_pages.data_ptr(),
             value_pages.data_ptr(), key_pages.stride(0), key_pages.stride(1),
@@ -1042,7 +1063,7 @@ def kv_append(k_new: torch.Tensor, v_new: torch.Tensor, key_pages: torch.Tensor,
     if v_new.stride(-1) != 1:
         v_new = v_new.contiguous()
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_paged_kv_append(
             k_new.data_ptr(), v_new.data_ptr(), _i64arr(k_new.stride()), _i64arr(v_new.stride()),
             key_pages.data_ptr(), value_pages.data_ptr(), key_pages.stride(0),
@@ -1092,7 +1113,7 @@ def _rope_kv_append(q, k, v, cos, sin, key_pages, value_pages, block_table, seq_
     sin = sin if sin.stride(-1) == 1 else sin.contiguous()
     q_out = torch.empty((B, Hq, S, D), dtype=q.dtype, device=dev)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_rope_kv_append(
             q.data_ptr(), _i64arr(q.stride()), k.data_ptr(), _i64arr(k.stride()), v.data_ptr(),
             _i64arr(v.stride()), q_out.data_ptr(), _i64arr(q_out.stride()), cos.data_ptr(),
@@ -1177,7 +1198,7 @@ def _paged_decode_step(q, k, v, cos, sin, key_pages, value_pages, block_table, s
     out = buf.transpose(1, 2)
     lse = torch.empty((B, Hq), dtype=torch.float32, device=dev) if return_lse else None
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_paged_decode_step(
             q.data_ptr(), q.stride(0), q.stride(1), k.data_ptr(), k.stride(0), k.stride(1),
             v.data_ptr(), v.stride(0), v.stride(1), cos.data_ptr(), sin.data_ptr(),
@@ -1206,7 +1227,7 @@ def kv_gather(key_pages: torch.Tensor, value_pages: torch.Tensor, block_table: t
     k_out = torch.empty((B, Hkv, length, D), dtype=key_pages.dtype, device=dev)
     v_out = torch.empty_like(k_out)
     lib = nat.load()
-    with _DeviceGuard(dev):
+    with _guard(dev):
         rc = lib.lc_paged_kv_gather(
             key_pages.data_ptr(), value_pages.data_ptr(), key_pages.stride(0),
             key_pages.stride(1), key_pages.stride(2), block_table.data_ptr(),

@@ -83,11 +83,12 @@ def _cuda_sdpa_causal_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tenso
 
 
 def _gqa_compatible(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> bool:
-    if q.dim() != 4 or k.dim() != 4 or v.dim() != 4 or k.shape != v.shape:
+    qs, ks = q.shape, k.shape
+    if len(qs) != 4 or len(ks) != 4 or ks != v.shape:
         return False
-    if q.shape[0] != k.shape[0] or q.shape[3] != k.shape[3]:
+    if qs[0] != ks[0] or qs[3] != ks[3]:
         return False
-    return k.shape[1] > 0 and q.shape[1] % k.shape[1] == 0
+    return ks[1] > 0 and qs[1] % ks[1] == 0
 
 
 def can_use_triton_fused_attention(
@@ -122,6 +123,8 @@ class _FusedCausalAttentionFunction(torch.autograd.Function):
         ctx.save_for_backward(q, k, v, out, lse, mask)
         ctx.q_offset = q_offset
         ctx.mark_non_differentiable(lse)
+        # (the lse's absent gradient is not filled with zeros for backward)
+        ctx.set_materialize_grads(False)
         return out, lse
 
     @staticmethod
