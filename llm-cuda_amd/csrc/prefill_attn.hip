@@ -40,17 +40,19 @@ struct PrefillArgs {
   int64_t bs[4];
   int bias_dtype;
   int bias_vec;
-  // Dynamic tail (no bias): a ticket that is zero at entry and left zero, and
-  // the lightest dyn_light row groups of each of the dyn_units units handed
-  // out through it; dyn_light == 0: every workgroup's item from its block id.
-  int* ticket;
-  int dyn_units, dyn_light;
   // Key splits (the SPLIT instances): n_splits ranges of split_tiles 64-key
   // tiles each; range z writes its normalised fp32 output to
   // ws_o[z][(b, h, i)][D] and its base-2 logsumexp to ws_l[z][(b, h, i)].
   float* ws_o;
   float* ws_l;
   int n_splits, split_tiles;
+  // (Last, beside the kernel's own arguments: every workgroup starts by loading
+  // them together.)
+  // Dynamic tail (no bias): a ticket that is zero at entry and left zero, and
+  // the lightest dyn_light row groups of each of the dyn_units units handed
+  // out through it; dyn_light == 0: every workgroup's item from its block id.
+  int* ticket;
+  int dyn_units, dyn_light;
 };
 
 // ---------------------------------------------------------------------------
