@@ -69,6 +69,23 @@ __device__ __forceinline__ int pf_snake(int q, int n) {
   return s < n ? s : q;
 }
 
+// Position of the q-th workgroup of an XCD in its heaviest-first list of n, for
+// a grid of more than one and at most two workgroups per CU, all of which start
+// at once: the ones that join a CU's first (from the pair_from-th on) run through
+// the rest of the list from its light end, so that a CU's two weigh about the
+// same. In list order the first CU gets the heaviest and the median one, 1.5
+// times the mean. Forward at 32/8 heads, D 128: [2, 1024] 36.6 -> 30.5 us, [4, 512]
+// 24.8 -> 22.0, [1, 2048] 47.9 -> 46.3; at 16/8, D 64: [2, 2048] 37.9 -> 31.1.
+__device__ __forceinline__ int pf_pair(int q, int n, int pair_from) {
+  return q < pair_from ? q : n - 1 - (q - pair_from);
+}
+// pair_from for a grid of nwg workgroups (a list order that suits any other
+// grid: none reversed).
+inline int pf_pair_from(int64_t nwg) {
+  const int cus = lc_cu_count();
+  return nwg % 8 == 0 && nwg > cus && nwg <= 2LL * cus ? cus / 8 : 0x7fffffff;
+}
+
 template <int CPR>
 __device__ __forceinline__ int pf_swz(int r) {
   if constexpr (CPR == 16) {

@@ -46,6 +46,7 @@ struct PrefillArgs {
   float* ws_o;
   float* ws_l;
   int n_splits, split_tiles;
+  int pair_from;  // see pf_pair
   // (Last, beside the kernel's own arguments: every workgroup starts by loading
   // them together.)
   // Dynamic tail (no bias): a ticket that is zero at entry and left zero, and
@@ -417,7 +418,8 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
     }
   } else {
     int work = lin;
-    if ((nwg & 7) == 0) work = (lin & 7) * (nwg >> 3) + (lin >> 3);
+    if ((nwg & 7) == 0)
+      work = (lin & 7) * (nwg >> 3) + pf_pair(lin >> 3, nwg >> 3, a.pair_from);
     unit = work / n_rbg;
     rbg = n_rbg - 1 - pf_snake(work - unit * n_rbg, n_rbg);
   }
@@ -1012,6 +1014,7 @@ int launch_mfma_split(PrefillArgs a, const PfGrid& g, int z, hipStream_t st) {
   a.n_splits = static_cast<int>((tiles + a.split_tiles - 1) / a.split_tiles);
   const int64_t rows = (int64_t)a.B * a.Hq * a.Sq;
   a.ws_l = a.ws_o + z * rows * a.D;
+  a.pair_from = 0x7fffffff;  // (at most one workgroup a CU)
   const int64_t nwg = g.nwg * a.n_splits;
   const int rpb = 256 / (a.D / 4);
   const int64_t mwg = (rows + rpb - 1) / rpb;
@@ -1026,7 +1029,7 @@ int launch_mfma_split(PrefillArgs a, const PfGrid& g, int z, hipStream_t st) {
 }
 
 template <typename T>
-int launch_mfma(const PrefillArgs& a, int64_t ws_bytes, hipStream_t st) {
+int launch_mfma(PrefillArgs a, int64_t ws_bytes, hipStream_t st) {
   const PfGrid g = pf_grid(a.B, a.Hq, a.Hkv, a.Sq);
   const int hw = g.hw, n_rbg = g.n_rbg;
   const int64_t nwg = g.nwg;
@@ -1037,6 +1040,7 @@ int launch_mfma(const PrefillArgs& a, int64_t ws_bytes, hipStream_t st) {
       return launch_mfma_split<T>(a, g, z, st);
   }
   dim3 grid(static_cast<unsigned>(nwg));
+  a.pair_from = pf_pair_from(nwg);
   // Dynamic tail: with a ticket, no bias, whole units per XCD (units a
   // multiple of 8), >= 8 row groups per unit and more than two rounds of
   // workgroups (two per CU). Measured at config 3 against the static order in

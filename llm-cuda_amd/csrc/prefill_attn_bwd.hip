@@ -63,6 +63,7 @@ struct BwdArgs {
   // of the blocks that have more than one leave fp32 sums in dkv_part.
   float* dkv_part;
   int dkv_share;
+  int pair_from;  // dQ: see pf_pair
 };
 
 // ---------------------------------------------------------------------------
@@ -725,7 +726,7 @@ attn_bwd_dq_mfma_kernel(BwdArgs a, int hw, int n_rbg) {
   const int nwg = gridDim.x;
   const int lin = blockIdx.x;
   int work = lin;
-  if ((nwg & 7) == 0) work = (lin & 7) * (nwg >> 3) + (lin >> 3);
+  if ((nwg & 7) == 0) work = (lin & 7) * (nwg >> 3) + pf_pair(lin >> 3, nwg >> 3, a.pair_from);
   const int unit = work / n_rbg;
   const int rbg = n_rbg - 1 - pf_snake(work - unit * n_rbg, n_rbg);
   const int kvh_hg = unit % (a.Hkv * n_hg);
@@ -1469,6 +1470,7 @@ int launch_bwd_mfma(BwdArgs a, int64_t part_bytes, hipStream_t st) {
   const int64_t nwg_k = (int64_t)n_kb * a.Hkv * a.B;
   LC_REQUIRE(nwg_q < (1LL << 31) && nwg_k < (1LL << 31), "lc_prefill_attn_bwd: grid too large");
   const int bias = a.bias == nullptr ? 0 : (a.bias_dtype == LC_DTYPE_F32 ? 2 : 1);
+  a.pair_from = bias == 0 ? pf_pair_from(nwg_q) : 0x7fffffff;  // (masked: one a CU)
   if (nwg_q > 0) {
     if (bias == 0)
       launch_dq_mfma<T, 0>(a, (unsigned)nwg_q, hw, n_rbg, st);
