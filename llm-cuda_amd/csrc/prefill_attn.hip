@@ -335,8 +335,9 @@ constexpr int kPrefillCounterInts = 64;
 // for every query row and head (the [B, 1, 1, Skv] padding masks) is staged in
 // LDS at the start, divided by scale_log2, and the S^T accumulators start from
 // it instead of from zero: no registers, no instructions per score, so it runs
-// two waves per SIMD. [8, 32/8, 1000, 128] with a padding mask: 108 us as 3,
-// 194 us as 1, 107 us unmasked.
+// two waves per SIMD. [8, 32/8, 1000, 128] with a left-padding mask: 96 us as
+// 3 (105 with the masked-away keys kept, 111 with an XCD to a sequence), 200 us
+// as 1, 105 us unmasked.
 //
 // SPLIT: one workgroup computes one key range of a row group (see
 // prefill_merge_kernel); the range's first key becomes key 0, so the keys
@@ -422,6 +423,12 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
       work = (lin & 7) * (nwg >> 3) + pf_pair(lin >> 3, nwg >> 3, a.pair_from);
     unit = work / n_rbg;
     rbg = n_rbg - 1 - pf_snake(work - unit * n_rbg, n_rbg);
+    if constexpr (BIAS == 3) {
+      // Sequences differ in how many keys their masks leave: an XCD takes every
+      // eighth unit, a share of each sequence, not one sequence's units.
+      const int per_xcd = nwg / n_rbg >> 3;
+      if (nwg == per_xcd * 8 * n_rbg) unit = unit % per_xcd * 8 + unit / per_xcd;
+    }
   }
   // Opaque from here on: the tile loop must not see which path chose them
   // (with both paths visible its register allocation grew past the budget).
@@ -443,6 +450,52 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   }
   const int kvh_hg = unit % (a.Hkv * n_hg);
   const int b = unit / (a.Hkv * n_hg);
+  // Key bias: staged, and the keys before the first and after the last one that
+  // is not masked away (bias at or below kBiasFloor, or -inf) left out for a
+  // workgroup whose every row sees that first one: their weight next to it is
+  // exactly 0. The first tile kept becomes tile 0, as in a split.
+  __shared__ __align__(16) float key_bias[BIAS == 3 ? kPfKeyBias : 4];
+  int bias0 = 0;  // first kept key, a multiple of a tile
+  if constexpr (BIAS == 3) {
+    // (in the V buffer that is filled only after the next barriers: two
+    // workgroups of this instance take all of a CU's LDS)
+    int* const s_lo = reinterpret_cast<int*>(lds_v1);
+    int* const s_hi = s_lo + kPfWaves;
+    const int vis = min(a.Skv, min(a.Sq - 1, (rbg + 1) * rbw * kPfRows - 1) + a.q_offset + 1);
+    const float inv = 1.0f / a.scale_log2;
+    int lo = 0x7fffffff, hi = -1;
+    for (int k0 = 0; k0 < vis; k0 += 64 * kPfWaves) {
+      const int k = k0 + tid;
+      // (the host passes at most kPfKeyBias visible keys)
+      const float x = k < vis ? lc_load_bias(a.bias, b * a.bs[0] + k * a.bs[3], a.bias_dtype)
+                              : -INFINITY;
+      if (k < vis) key_bias[k] = lc_bias_log2(x) * inv;
+      const uint64_t kept = __ballot(x > kBiasFloor);
+      if (kept != 0) {
+        lo = min(lo, k0 + wave_s * 64 + __builtin_ctzll(kept));
+        hi = max(hi, k0 + wave_s * 64 + 63 - __builtin_clzll(kept));
+      }
+    }
+    if (lane == 0) {
+      s_lo[wave] = lo;
+      s_hi[wave] = hi;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int w = 0; w < kPfWaves; ++w) {
+      lo = min(lo, s_lo[w]);
+      hi = max(hi, s_hi[w]);
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
+    if (rbg * rbw * kPfRows + a.q_offset >= lo) {
+      bias0 = lo / kPfKeys * kPfKeys;
+      a.k = static_cast<const T*>(a.k) + bias0 * a.ks[2];
+      a.v = static_cast<const T*>(a.v) + bias0 * a.vs[2];
+      a.Skv = hi + 1 - bias0;
+      a.q_offset -= bias0;
+    }
+  }
   const int kvh = kvh_hg / n_hg;
   const int hgi = kvh_hg - kvh * n_hg;
   const int head = kvh * a.G + hgi * hw + (wave % hw);
@@ -482,15 +535,6 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   auto load_bias = [&](int t) __attribute__((always_inline)) {
     if constexpr (ROW_BIAS) btile.load(brs, brow_b, t * kPfKeys, hh, bs3_b, a.bias_vec != 0);
   };
-  __shared__ __align__(16) float key_bias[BIAS == 3 ? kPfKeyBias : 4];
-  if constexpr (BIAS == 3) {
-    // (the host passes at most kPfKeyBias visible keys; published by the barrier
-    // before the first scores)
-    const float inv = 1.0f / a.scale_log2;
-    for (int k = tid; k < kv_end; k += 64 * kPfWaves)
-      key_bias[k] =
-          lc_bias_log2(lc_load_bias(a.bias, b * a.bs[0] + k * a.bs[3], a.bias_dtype)) * inv;
-  }
 
   // Q^T operand registers.
   v8 qop[KS];
@@ -579,7 +623,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           const f32x4_t b4 = *reinterpret_cast<LC_LDS const f32x4_t*>(
-              (LC_LDS const float*)key_bias + k0 + kt * 32 + j * 8 + hh * 4);
+              (LC_LDS const float*)key_bias + bias0 + k0 + kt * 32 + j * 8 + hh * 4);
 #pragma unroll
           for (int i = 0; i < 4; ++i) snx[kt][j * 4 + i] = b4[i];
         }

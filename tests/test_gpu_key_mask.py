@@ -66,6 +66,35 @@ def test_key_mask(cuda, kind, Sq, Skv, D, dtype, mdt):
         assert (out.double() - _reference(q, k, v, mask, off)).abs().max().item() <= ATOL[dtype]
 
 
+@pytest.mark.parametrize("value", ["min", -math.inf])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D", [
+    (3, 8, 2, 400, 400, 128),   # 6 units: the plain unit order
+    (2, 16, 8, 300, 450, 64),   # 16 units dealt over the XCDs, a cached prefix
+])
+def test_masked_ends_are_left_out(cuda, value, B, Hq, Hkv, Sq, Skv, D):
+    """Padding of several tiles at both ends: rows before, on and after the kept
+    keys, a sequence with one kept key and one with none masked."""
+    from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
+
+    dtype, off = torch.bfloat16, Skv - Sq
+    g = torch.Generator().manual_seed(Skv)
+    q, k, v = (torch.randn(s, generator=g).to(dtype).to(cuda) for s in (
+        (B, Hq, Sq, D), (B, Hkv, Skv, D), (B, Hkv, Skv, D)))
+    mask = torch.zeros(B, 1, 1, Skv)
+    low = torch.finfo(dtype).min if value == "min" else value
+    mask[0, ..., :197] = mask[0, ..., 330:] = low
+    mask[1] = low
+    mask[1, ..., 131] = 0.25
+    mask = mask.to(dtype).to(cuda)
+    out, lse = triton_fused_causal_attention(q, k, v, mask, return_lse=True, q_offset=off)
+    assert (out.double() - _reference(q, k, v, mask, off)).abs().max().item() <= ATOL[dtype]
+    rows, rlse = triton_fused_causal_attention(
+        q, k, v, mask.expand(B, 1, Sq, Skv).contiguous(), return_lse=True, q_offset=off)
+    assert torch.equal(torch.isinf(lse), torch.isinf(rlse))
+    real = torch.isfinite(lse)
+    assert ((lse - rlse)[real].abs() <= 1e-5 + 2.0 ** -21 * rlse[real].abs()).all()
+
+
 @pytest.mark.parametrize("Skv", [4096, 4097])
 def test_key_mask_at_the_most_keys_staged(cuda, Skv):
     from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
