@@ -133,8 +133,9 @@ LC_API int lc_rope_fwd(const void* x1, void* out1, int64_t h1, const int64_t* x1
  * row whose visible keys are all so masked averages them, as the reference's
  * softmax of equal scores does; -inf excludes a key, and a row without any
  * visible key gives o = 0, lse = -inf (the reference gives NaN there).
- * Hq % Hkv == 0. bf16/f16 run on MFMA (D in {64, 128}); other cases run a
- * generic fp32-FMA kernel (D <= 256).
+ * Hq % Hkv == 0. bf16/f16 (D a multiple of 8 up to 128) and fp32 (D a multiple
+ * of 4 up to 128) run on MFMA; other cases run a generic fp32-FMA kernel
+ * (D <= 256).
  * counters: lc_prefill_attn_counter_count() int32 values that are zero at
  *   entry and are left zero, or NULL. With counters, the MFMA kernel hands the
  *   lightest quarter of its row groups out to the workgroups in the order they

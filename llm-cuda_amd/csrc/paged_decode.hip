@@ -7,8 +7,9 @@
 // decode kernel re-read K/V once per query head:
 // kernels/triton/decode_attention.py:86-93,110-151).
 //
-// Main kernel (page_size a multiple of 32), per 32-token step:
-//   1. the step's K and V rows (one page, so the page id is wave-uniform) are
+// Main kernel (page_size a multiple of 32, or 16), per 32-token step:
+//   1. the step's K and V rows (one page, so the page id is wave-uniform; a page
+//      per half step at 16) are
 //      read with fully coalesced 16-byte buffer loads (16 lanes per 256-byte
 //      row) carrying the non-temporal hint, into one register staging buffer;
 //   2. the staging buffer is copied to wave-private LDS tiles and the NEXT
@@ -1012,7 +1013,8 @@ __global__ __launch_bounds__(64 * cluster_waves<DPAD>()) void paged_decode_clust
   }
 }
 
-// Page sizes that are not multiples of 32: per-lane page resolution.
+// Page sizes that are neither 16 nor multiples of 32 (and masked or one-wave
+// splits of 16): per-lane page resolution.
 // Three waves per SIMD up to head_dim 128: at 144 VGPRs and 9 KiB of LDS the
 // kernel fits them without spills, and the extra loads in flight measured 6%
 // faster than two. (head_dim 256 would spill at three.)

@@ -735,10 +735,14 @@ def decode_linear_partials(x: torch.Tensor, weight: torch.Tensor, shares: int = 
 # Small fp32 projections  (reference: the nn.Linear calls of an fp32 model,
 # models/llama3/attention.py:100-102,154 and mlp.py:35-43)
 # ---------------------------------------------------------------------------
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
 def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """True where linear_f32 takes a projection over from the library's GEMM:
     fp32 on the GPU, K <= 768, at most 256 tiles of 32 x 32 outputs, no autograd
-    graph being recorded, no autocast, and not inside torch_projections().
+    graph being recorded, no autocast, plain tensors, and not inside
+    torch_projections().
 
     The line: one round of the CUs and a K that eight waves contract in a few
     microseconds. Graph-replayed us a call, here / library: K 256, N 512, 64
@@ -746,6 +750,8 @@ def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
     tiles, K 688 6.7 / 160, K 1024 10.6 / 6.0; N 384, K 384 5.8 / 5.4 (the
     library's call costs 13 us more on the host)."""
     if not _NATIVE_PROJECTIONS[0] or not (x.is_cuda and weight.is_cuda):
+        return False
+    if type(x) not in _PLAIN or type(weight) not in _PLAIN:  # (a subclass has its own linear)
         return False
     if not (x.dtype == weight.dtype == torch.float32 and weight.dim() == 2 and x.dim() >= 1):
         return False
