@@ -61,6 +61,24 @@ def test_f32_attention_matches_float64(cuda, B, Hq, Hkv, Sq, Skv, D):
     _check(_run(q, k, v, do, Skv - Sq), _reference(q, k, v, do, Skv - Sq, None), D, Skv)
 
 
+@pytest.mark.parametrize("D", [20, 64, 128])
+def test_f32_attention_layouts(cuda, D):
+    """Rows of odd strides from an odd element on (4-byte aligned only), projection
+    views, a batch that shares its keys (stride 0), and a strided gradient."""
+    B, Hq, Hkv, S = 2, 4, 2, 70
+    g = torch.Generator().manual_seed(D)
+    q = torch.randn(B, Hq, S, D + 3, generator=g).to(cuda)[..., 1:D + 1]
+    k = torch.randn(1, Hkv, S, D + 5, generator=g).to(cuda)[..., 3:D + 3].expand(B, -1, -1, -1)
+    v = torch.randn(B, S, Hkv, D, generator=g).to(cuda).transpose(1, 2)
+    do = torch.randn(B, S, Hq, D + 1, generator=g).to(cuda)[..., 1:].transpose(1, 2)
+    from llm_cuda.kernels import _ops
+
+    out, lse = _ops.prefill_attention(q, k, v, return_lse=True)
+    grads = _ops.prefill_attention_backward(q, k, v, out, lse, do)
+    ref = _reference(q, k, v, do, 0, None)
+    _check((out, lse, *grads), ref, D, S)
+
+
 @pytest.mark.parametrize("D", [32, 64, 128])
 def test_f32_attention_with_mask(cuda, D):
     B, H, S = 2, 4, 150

@@ -66,6 +66,26 @@ def test_key_mask(cuda, kind, Sq, Skv, D, dtype, mdt):
         assert (out.double() - _reference(q, k, v, mask, off)).abs().max().item() <= ATOL[dtype]
 
 
+@pytest.mark.parametrize("form", ["batch of one", "every other", "one value", "odd start"])
+def test_key_mask_forms(cuda, form):
+    """Masks that broadcast or stride: one for the batch, a strided row, a single
+    value for every key, rows from an odd element on; views of q, k and v."""
+    from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
+
+    B, Hq, Hkv, S, D, dtype = 2, 8, 2, 150, 64, torch.bfloat16
+    g = torch.Generator().manual_seed(1)
+    q, k, v = (torch.randn(B, S, h, D, generator=g).to(dtype).to(cuda).transpose(1, 2)
+               for h in (Hq, Hkv, Hkv))
+    m = torch.zeros(B, 1, 1, 2 * S + 1, dtype=dtype, device=cuda)
+    m[0, ..., :80] = torch.finfo(dtype).min
+    m[1, ..., ::3] = -2.5
+    mask = {"batch of one": m[:1, ..., :S], "every other": m[..., :2 * S:2],
+            "one value": m[1:, ..., :1], "odd start": m[..., 1:S + 1]}[form]
+    out = triton_fused_causal_attention(q, k, v, mask)
+    ref = _reference(q, k, v, mask.expand(B, 1, 1, S), 0)
+    assert (out.double() - ref).abs().max().item() <= ATOL[dtype]
+
+
 @pytest.mark.parametrize("value", ["min", -math.inf])
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Skv,D", [
     (3, 8, 2, 400, 400, 128),   # 6 units: the plain unit order

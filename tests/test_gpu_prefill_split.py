@@ -67,6 +67,22 @@ def test_split_prefill(cuda, B, Hq, Hkv, Sq, Skv, off, D, dtype):
     assert (out.float() - out1.float()).abs().max().item() <= ATOL[dtype]
 
 
+def test_split_prefill_strided_views(cuda):
+    """q, k and v as projection views, k and v cut from longer rows, a batch that
+    shares its keys."""
+    from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
+
+    B, Hq, Hkv, Sq, Skv, D = 2, 8, 2, 50, 2200, 64
+    g = torch.Generator().manual_seed(4)
+    q = torch.randn(B, Sq, Hq, D, generator=g).bfloat16().to(cuda).transpose(1, 2)
+    kv = torch.randn(1, Skv, 2 * Hkv, D + 8, generator=g).bfloat16().to(cuda).transpose(1, 2)
+    k, v = (t[..., 8:].expand(B, -1, -1, -1) for t in (kv[:, :Hkv], kv[:, Hkv:]))
+    out, lse = triton_fused_causal_attention(q, k, v, return_lse=True, q_offset=Skv - Sq)
+    ref, rlse = _unsplit(q.contiguous(), k.contiguous(), v.contiguous(), Skv - Sq)
+    assert (lse - rlse).abs().max().item() <= Skv * 2.0 ** -23 + 1e-5
+    assert (out.float() - ref.float()).abs().max().item() <= ATOL[torch.bfloat16]
+
+
 def test_split_prefill_replays_from_a_graph(cuda):
     from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
 
