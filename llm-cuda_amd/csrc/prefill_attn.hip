@@ -333,11 +333,14 @@ constexpr int kPrefillCounterInts = 64;
 // (1, 2) the kernel runs one wave per SIMD: the bias tile held one iteration
 // ahead does not fit the two-wave register budget without spills. A bias alike
 // for every query row and head (the [B, 1, 1, Skv] padding masks) is staged in
-// LDS at the start, divided by scale_log2, and the S^T accumulators start from
-// it instead of from zero: no registers, no instructions per score, so it runs
-// two waves per SIMD. [8, 32/8, 1000, 128] with a left-padding mask: 96 us as
-// 3 (105 with the masked-away keys kept, 111 with an XCD to a sequence), 200 us
-// as 1, 105 us unmasked.
+// LDS at the start and read there, four keys at a time, by the SM1 that adds it
+// with the scale's own fma: no registers held across the tile, so it runs two
+// waves per SIMD (233 VGPRs at D = 128). The arithmetic is that of 1 and 2,
+// bit for bit. (Starting the S^T accumulators from bias / scale instead rounds
+// at the bias's size in every k-step and gives lses of masked rows that the
+// backward does not meet again; it is no faster: 98 us below.)
+// [8, 32/8, 1000, 128] with a left-padding mask: 96 us as 3, 200 us as 1, 105 us
+// unmasked.
 //
 // SPLIT: one workgroup computes one key range of a row group (see
 // prefill_merge_kernel); the range's first key becomes key 0, so the keys
@@ -462,14 +465,13 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
     int* const s_lo = reinterpret_cast<int*>(lds_v1);
     int* const s_hi = s_lo + kPfWaves;
     const int vis = min(a.Skv, min(a.Sq - 1, (rbg + 1) * rbw * kPfRows - 1) + a.q_offset + 1);
-    const float inv = 1.0f / a.scale_log2;
     int lo = 0x7fffffff, hi = -1;
     for (int k0 = 0; k0 < vis; k0 += 64 * kPfWaves) {
       const int k = k0 + tid;
       // (the host passes at most kPfKeyBias visible keys)
       const float x = k < vis ? lc_load_bias(a.bias, b * a.bs[0] + k * a.bs[3], a.bias_dtype)
                               : -INFINITY;
-      if (k < vis) key_bias[k] = lc_bias_log2(x) * inv;
+      if (k < vis) key_bias[k] = lc_bias_log2(x);
       const uint64_t kept = __ballot(x > kBiasFloor);
       if (kept != 0) {
         lo = min(lo, k0 + wave_s * 64 + __builtin_ctzll(kept));
@@ -611,23 +613,11 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
     return wave_active && t < n_tiles && t * kPfKeys < my_kv_end;
   };
 
-  auto qk = [&](LC_LDS const char* kt_lds, int k0) __attribute__((always_inline)) {
+  auto qk = [&](LC_LDS const char* kt_lds) __attribute__((always_inline)) {
 #pragma unroll
     for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
       for (int r = 0; r < 16; ++r) snx[kt][r] = 0.f;
-    if constexpr (BIAS == 3) {
-      // (what keys past kv_end read is masked)
-#pragma unroll
-      for (int kt = 0; kt < 2; ++kt)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const f32x4_t b4 = *reinterpret_cast<LC_LDS const f32x4_t*>(
-              (LC_LDS const float*)key_bias + bias0 + k0 + kt * 32 + j * 8 + hh * 4);
-#pragma unroll
-          for (int i = 0; i < 4; ++i) snx[kt][j * 4 + i] = b4[i];
-        }
-    }
     // The two 32-key halves alternate, so consecutive MFMAs are independent.
 #pragma unroll
     for (int s = 0; s < KS; ++s)
@@ -655,16 +645,22 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   // SM1 of the tile whose raw scores are in snx (keys k0 ..): sets xcu, the
   // running max and row sum; a required rescale of O is left to apply_rescale.
   auto sm1 = [&](int k0, auto mask_c) __attribute__((always_inline)) {
-    // (no fused s * scale - m: at a masked row's m of -1e30 its one rounding
-    // differs from m's by far more than 1)
-#pragma clang fp contract(off)
+    // Scores with the bias, in the exp2 domain: one rounding of the exact-size
+    // product next to the bias, and the value that the backward adds, so that a
+    // row whose keys are all masked gets an lse that the backward meets again.
     if constexpr (BIAS == 3) {
+      // (what keys past kv_end read is masked)
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) snx[kt][r] *= a.scale_log2;
+        for (int j = 0; j < 4; ++j) {
+          const f32x4_t b4 = *reinterpret_cast<LC_LDS const f32x4_t*>(
+              (LC_LDS const float*)key_bias + bias0 + k0 + kt * 32 + j * 8 + hh * 4);
+#pragma unroll
+          for (int i = 0; i < 4; ++i)
+            snx[kt][j * 4 + i] = fmaf(snx[kt][j * 4 + i], a.scale_log2, b4[i]);
+        }
     } else if constexpr (BIAS != 0) {
-      // Scores with the bias, in the exp2 domain.
 #pragma unroll
       for (int kt = 0; kt < 2; ++kt)
 #pragma unroll
@@ -813,7 +809,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
     if constexpr (BIAS == 0) {
       if (cur && nxt) {
         constexpr int NQ = 2 * KS, NP = 4 * DTL, LA = 4;
-        qk(kbuf(other), k1);
+        qk(kbuf(other));
         sm2l();
         __builtin_amdgcn_sched_group_barrier(0x100, LA, 0);
 #pragma unroll
@@ -833,7 +829,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
           __builtin_amdgcn_sched_group_barrier(0x002, 2, 0);
         }
       } else {
-        if (nxt) qk(kbuf(other), k1);
+        if (nxt) qk(kbuf(other));
         if (cur) {
           sm2l();
           check_fix();
@@ -845,7 +841,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
       return;
     }
     if (cur && nxt) {
-      qk(kbuf(other), k1);
+      qk(kbuf(other));
       sm2();
       pv(vbuf(par_c));
       sm1(k1, mask_c);
@@ -853,7 +849,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
       // SM2 VALU work; part B: 16 PV MFMAs, each with two V^T reads ahead
       // and SM1 VALU work.
       constexpr int NQ = 2 * KS, NP = 4 * DTL, LA = 4;
-      __builtin_amdgcn_sched_group_barrier(0x100, LA + (BIAS == 3 ? 8 : 0), 0);
+      __builtin_amdgcn_sched_group_barrier(0x100, LA, 0);
 #pragma unroll
       for (int j = 0; j < NQ + NP; ++j) {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -862,10 +858,13 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
           __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         else if (nx < NQ + NP)
           __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        // (four keys' bias a step, two steps ahead of the SM1 work that adds it)
+        if (BIAS == 3 && j + 2 >= NQ && j + 2 < NQ + 8)
+          __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
         __builtin_amdgcn_sched_group_barrier(0x002, 4, 0);
       }
     } else {
-      if (nxt) qk(kbuf(other), k1);
+      if (nxt) qk(kbuf(other));
       if (cur) {
         sm2();
         pv(vbuf(par_c));
@@ -889,7 +888,7 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   if (live(0)) load_bias(0);
   pf_barrier<true>();
   if (live(0)) {
-    qk(kbuf(std::integral_constant<int, 0>{}), 0);
+    qk(kbuf(std::integral_constant<int, 0>{}));
     sm1(0, std::true_type{});
     rescale = false;  // O is still zero
   }
@@ -1103,10 +1102,9 @@ int launch_mfma(PrefillArgs a, int64_t ws_bytes, hipStream_t st) {
   } else if (a.bias == nullptr)
     launch_mfma_bias<T, 0>(a, grid, hw, n_rbg, st);
   else if (a.bs[1] == 0 && a.bs[2] == 0 && (int64_t)a.Sq + a.q_offset < (1LL << 31) &&
-           min(a.Skv, a.Sq + a.q_offset) <= kPfKeyBias && a.scale_log2 > 1e-6f &&
-           a.scale_log2 < 1e6f)
-    // A key bias (see the kernel); a scale that its division cannot take, or
-    // more keys than LDS holds, leaves it to the row-bias instances.
+           min(a.Skv, a.Sq + a.q_offset) <= kPfKeyBias)
+    // A key bias (see the kernel); more keys than LDS holds leave it to the
+    // row-bias instances.
     launch_mfma_bias<T, 3>(a, grid, hw, n_rbg, st);
   else if (a.bias_dtype == LC_DTYPE_F32)
     launch_mfma_bias<T, 2>(a, grid, hw, n_rbg, st);
