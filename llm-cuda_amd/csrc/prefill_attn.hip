@@ -923,10 +923,14 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
   if (qi >= a.Sq) return;
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   if constexpr (SPLIT) {
-    // (the merge reads no output of a range without visible keys)
+    // A row that sees no key of the range (its shifted offset is below zero) is
+    // marked by -inf, and the merge reads none of its output. Decided from the
+    // indices: a row sum of NaN, or of scores that are all -inf, is a result,
+    // which the merge carries on.
+    const bool seen = qi + a.q_offset >= 0;
     const int64_t row = split_row + ((int64_t)b * a.Hq + head) * a.Sq + qi;
     float* prow = a.ws_o + row * a.D;
-    if (l_tot > 0.f) {
+    if (seen) {
 #pragma unroll
       for (int dt = 0; dt < DTL; ++dt)
 #pragma unroll
@@ -940,7 +944,8 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
           }
         }
     }
-    if (hh == 0) a.ws_l[row] = l_tot > 0.f ? m_ref + lc_log2(l_tot) : -INFINITY;
+    if (hh == 0)  // (log2 of a NaN sum is NaN; of 0 it is -inf)
+      a.ws_l[row] = seen ? (l_tot == 0.f ? -INFINITY : m_ref + lc_log2(l_tot)) : -INFINITY;
     return;
   }
   T* orow = static_cast<T*>(a.o) + b * a.os[0] + (int64_t)head * a.os[1] + (int64_t)qi * a.os[2];
@@ -963,7 +968,8 @@ prefill_mfma_kernel(PrefillArgs a, int hw, int n_rbg) {
 }
 
 // Combines the key ranges of SPLIT launches: o = sum_z 2^(l_z - L) o_z with
-// L = log2 sum_z 2^(l_z). D / 4 lanes a row, 16 bytes of each range per lane;
+// L = log2 sum_z 2^(l_z). A range whose l_z is NaN makes the row NaN (and its
+// lse -inf), as it does without a split. D / 4 lanes a row, 16 bytes of each range per lane;
 // bound by reading the fp32 partials once (they are mostly still in L2).
 template <typename T>
 __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int64_t rows) {
@@ -977,14 +983,13 @@ __global__ __launch_bounds__(256) void prefill_merge_kernel(PrefillArgs a, int64
   for (int z = 0; z < a.n_splits; ++z) m = fmaxf(m, a.ws_l[z * rows + row]);
   float l = 0.f;
   f32x4_t acc = {0.f, 0.f, 0.f, 0.f};
-  if (m != -INFINITY) {
-    for (int z = 0; z < a.n_splits; ++z) {
-      const float lz = a.ws_l[z * rows + row];
-      if (lz == -INFINITY) continue;  // no visible key: nothing was written
-      const float w = lc_exp2(lz - m);
-      l += w;
-      acc += *reinterpret_cast<const f32x4_t*>(a.ws_o + (z * rows + row) * a.D + d) * w;
-    }
+  for (int z = 0; z < a.n_splits; ++z) {
+    const float lz = a.ws_l[z * rows + row];
+    if (lz == -INFINITY) continue;  // no visible key: nothing was written
+    // (m, a maximum that passes over NaN, is -inf where every other range is)
+    const float w = lc_exp2(lz - m);
+    l += w;
+    acc += *reinterpret_cast<const f32x4_t*>(a.ws_o + (z * rows + row) * a.D + d) * w;
   }
   const float inv = l > 0.f ? 1.0f / l : 0.f;
   const int i = static_cast<int>(row % a.Sq);

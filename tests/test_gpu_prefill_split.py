@@ -99,3 +99,26 @@ def test_split_prefill_replays_from_a_graph(cuda):
         torch.cuda.synchronize()
         assert all(torch.equal(a, b) for a, b in zip(got, ref))
         run()
+
+
+# A NaN or inf in one K row of a range (seen by all rows; by the last 20 only; in
+# the first and in the last tile of a range), in one element of V, in a Q row.
+@pytest.mark.parametrize("where,value", [
+    ("k 1000", math.nan), ("k 2980", math.nan), ("k 0", math.nan), ("k 511", math.nan),
+    ("k 1000", math.inf), ("v 700", math.nan), ("q 7", math.nan), ("q 7", math.inf)])
+def test_split_prefill_keeps_what_is_not_finite(cuda, where, value):
+    from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
+
+    B, Hq, Hkv, Sq, Skv, D = 1, 8, 2, 40, 3000, 128
+    q, k, v = _inputs(B, Hq, Hkv, Sq, Skv, D, torch.bfloat16, cuda)
+    name, row = where.split()
+    if name == "v":
+        v[0, 1, int(row), 3] = value
+    else:
+        dict(q=q, k=k)[name][0, 1, int(row)] = value
+    out, lse = triton_fused_causal_attention(q, k, v, return_lse=True, q_offset=Skv - Sq)
+    ref, rlse = _unsplit(q, k, v, Skv - Sq)
+    assert not ref.isfinite().all()
+    assert torch.equal(out.isnan(), ref.isnan()) and torch.equal(lse.isinf(), rlse.isinf())
+    fine = ref.isfinite()
+    assert (out.float() - ref.float())[fine].abs().max().item() <= ATOL[torch.bfloat16]
