@@ -1088,7 +1088,16 @@ int launch_mfma(PrefillArgs a, int64_t ws_bytes, hipStream_t st) {
       return launch_mfma_split<T>(a, g, z, st);
   }
   dim3 grid(static_cast<unsigned>(nwg));
-  a.pair_from = pf_pair_from(nwg);
+  // A key bias (see the kernel); more keys than LDS holds leave it to the
+  // row-bias instances.
+  const bool key_bias = a.bias != nullptr && a.bs[1] == 0 && a.bs[2] == 0 &&
+                        (int64_t)a.Sq + a.q_offset < (1LL << 31) &&
+                        min(a.Skv, a.Sq + a.q_offset) <= kPfKeyBias;
+  // The row-bias instances run one workgroup per CU: past the first round of
+  // them the rest start one by one, heaviest first as in any longer grid (with
+  // pairs [2, 1000] at 32/8 heads, D 128, takes 73 us instead of 53, [1, 2048]
+  // 120 instead of 97).
+  a.pair_from = a.bias == nullptr || key_bias ? pf_pair_from(nwg) : 0x7fffffff;
   // Dynamic tail: with a ticket, no bias, whole units per XCD (units a
   // multiple of 8), >= 8 row groups per unit and more than two rounds of
   // workgroups (two per CU). Measured at config 3 against the static order in
@@ -1106,10 +1115,7 @@ int launch_mfma(PrefillArgs a, int64_t ws_bytes, hipStream_t st) {
     launch_mfma_bias<T, 0>(d, dim3(static_cast<unsigned>(nwg + spare)), hw, n_rbg, st);
   } else if (a.bias == nullptr)
     launch_mfma_bias<T, 0>(a, grid, hw, n_rbg, st);
-  else if (a.bs[1] == 0 && a.bs[2] == 0 && (int64_t)a.Sq + a.q_offset < (1LL << 31) &&
-           min(a.Skv, a.Sq + a.q_offset) <= kPfKeyBias)
-    // A key bias (see the kernel); more keys than LDS holds leave it to the
-    // row-bias instances.
+  else if (key_bias)
     launch_mfma_bias<T, 3>(a, grid, hw, n_rbg, st);
   else if (a.bias_dtype == LC_DTYPE_F32)
     launch_mfma_bias<T, 2>(a, grid, hw, n_rbg, st);
