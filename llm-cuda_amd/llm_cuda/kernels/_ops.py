@@ -801,13 +801,26 @@ def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return F.linear(x, weight)
 
 
-def project(x: torch.Tensor, module: torch.nn.Module) -> torch.Tensor:
-    """module(x) for a projection; a plain bias-free nn.Linear without hooks runs
-    as linear_f32 where that applies."""
-    if (type(module) is torch.nn.Linear and module.bias is None
+_LINEAR_FORWARD = torch.nn.Linear.forward
+
+
+def _is_plain_linear(module: torch.nn.Module) -> bool:
+    """Whether module(x) is F.linear(x, module.weight) and nothing else: an
+    nn.Linear itself without bias, hooks or a compiled call, whose forward nobody
+    replaced (on the instance, as wrappers and quantisers do, or on the class)."""
+    return (type(module) is torch.nn.Linear and module.bias is None
+            and "forward" not in module.__dict__ and torch.nn.Linear.forward is _LINEAR_FORWARD
+            and module._compiled_call_impl is None
             and not (module._forward_hooks or module._forward_pre_hooks
-                     or _module._global_forward_hooks or _module._global_forward_pre_hooks)
-            and linear_f32_applies(x, module.weight)):
+                     or module._backward_hooks or module._backward_pre_hooks
+                     or _module._global_forward_hooks or _module._global_forward_pre_hooks
+                     or _module._global_backward_hooks or _module._global_backward_pre_hooks))
+
+
+def project(x: torch.Tensor, module: torch.nn.Module) -> torch.Tensor:
+    """module(x) for a projection; a plain nn.Linear (see _is_plain_linear) runs as
+    linear_f32 where that applies."""
+    if _is_plain_linear(module) and linear_f32_applies(x, module.weight):
         return linear_f32(x, module.weight)
     return module(x)
 

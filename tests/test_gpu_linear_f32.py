@@ -46,3 +46,24 @@ def test_linear_f32_leaves_other_calls_to_torch(cuda):
     lin = torch.nn.Linear(64, 32, bias=False, device=cuda).requires_grad_(False)
     lin.register_forward_hook(lambda m, i, o: o + 1)
     assert torch.equal(_ops.project(x, lin), F.linear(x, lin.weight) + 1)
+
+
+@pytest.mark.parametrize("where", ["instance", "class", "backward hook"])
+def test_project_calls_what_replaced_the_forward(cuda, where, monkeypatch):
+    """A wrapper's own forward (offloading, adapters, quantisation) runs."""
+    from llm_cuda.kernels import _ops
+
+    x = torch.randn(4, 64, device=cuda)
+    lin = torch.nn.Linear(64, 32, bias=False, device=cuda).requires_grad_(False)
+    assert torch.equal(_ops.project(x, lin), _ops.linear_f32(x, lin.weight))
+    if where == "backward hook":
+        lin.register_full_backward_hook(lambda m, gi, go: None)
+        assert not _ops._is_plain_linear(lin)
+        return
+    plain = F.linear(x, lin.weight)
+    if where == "instance":
+        own = lin.forward
+        lin.forward = lambda t: own(t) + 1
+    else:
+        monkeypatch.setattr(torch.nn.Linear, "forward", lambda m, t: F.linear(t, m.weight) + 1)
+    assert torch.equal(_ops.project(x, lin), plain + 1)
