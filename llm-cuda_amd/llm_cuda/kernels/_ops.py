@@ -14,6 +14,7 @@ import math
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad as _forward_ad
 from torch.nn.modules import module as _module
 
 from llm_cuda import _native as nat
@@ -738,11 +739,22 @@ def decode_linear_partials(x: torch.Tensor, weight: torch.Tensor, shares: int = 
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
 
 
+def _watched() -> bool:
+    """Whether something beside autograd follows torch's calls and would miss a
+    native launch: a function or dispatch mode (FLOP counters, fake tensors), a
+    functorch transform (vmap, jvp), a trace, or a forward-mode level, whose
+    tangents F.linear carries."""
+    return (torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
+            or torch._C._functorch.maybe_current_level() is not None
+            or _forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
+            or torch.compiler.is_compiling())
+
+
 def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """True where linear_f32 takes a projection over from the library's GEMM:
     fp32 on the GPU, K <= 768, at most 256 tiles of 32 x 32 outputs, no autograd
-    graph being recorded, no autocast, plain tensors, and not inside
-    torch_projections().
+    graph being recorded, no autocast, plain tensors, nothing that follows
+    torch's calls (see _watched), and not inside torch_projections().
 
     The line: one round of the CUs and a K that eight waves contract in a few
     microseconds. Graph-replayed us a call, here / library: K 256, N 512, 64
@@ -761,7 +773,7 @@ def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
     rows = x.numel() // K
     if not 0 < -(-rows // 32) * -(-N // 32) <= 256:
         return False
-    if _records_grad(x, weight) or torch.is_autocast_enabled():
+    if _records_grad(x, weight) or torch.is_autocast_enabled() or _watched():
         return False
     return weight.stride(1) == 1 and (N == 1 or K <= weight.stride(0) < 2 ** 23)
 

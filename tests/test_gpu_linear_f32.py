@@ -67,3 +67,36 @@ def test_project_calls_what_replaced_the_forward(cuda, where, monkeypatch):
     else:
         monkeypatch.setattr(torch.nn.Linear, "forward", lambda m, t: F.linear(t, m.weight) + 1)
     assert torch.equal(_ops.project(x, lin), plain + 1)
+
+
+def test_linear_stays_with_torch_where_its_calls_are_followed(cuda):
+    """Forward-mode tangents, FLOP counters, function modes, vmap and traces."""
+    from torch.autograd import forward_ad
+    from torch.utils.flop_counter import FlopCounterMode
+
+    from llm_cuda.kernels import _ops
+
+    x, w, t = (torch.randn(s, 64, device=cuda) for s in (4, 32, 32))
+    assert _ops.linear_f32_applies(x, w)
+    with forward_ad.dual_level():
+        tangent = forward_ad.unpack_dual(_ops.linear(x, forward_ad.make_dual(w, t))).tangent
+        assert torch.equal(tangent, F.linear(x, t))
+    with FlopCounterMode(display=False) as flops:
+        _ops.linear(x, w)
+    assert flops.get_total_flops() == 2 * 4 * 32 * 64
+
+    class Seen(torch.overrides.TorchFunctionMode):
+        calls = []
+
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            self.calls.append(func)
+            return func(*args, **(kwargs or {}))
+
+    with Seen():
+        _ops.linear(x, w)
+    assert F.linear in Seen.calls
+    xs = torch.stack((x, 2 * x))
+    assert torch.allclose(torch.func.vmap(lambda u: _ops.linear(u, w))(xs), F.linear(xs, w))
+    traced = torch.jit.trace(lambda u: _ops.linear(u, w), x)
+    assert torch.allclose(traced(3 * x), F.linear(3 * x, w), atol=1e-4)
+    assert _ops.linear_f32_applies(x, w)
