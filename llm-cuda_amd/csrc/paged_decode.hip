@@ -1013,7 +1013,7 @@ __global__ __launch_bounds__(64 * cluster_waves<DPAD>()) void paged_decode_clust
   }
 }
 
-// Page sizes that are neither 16 nor multiples of 32 (and masked or one-wave
+// Page sizes that are neither 16 nor multiples of 32 (and masked, short or one-wave
 // splits of 16): per-lane page resolution.
 // Three waves per SIMD up to head_dim 128: at 144 VGPRs and 9 KiB of LDS the
 // kernel fits them without spills, and the extra loads in flight measured 6%
@@ -1386,6 +1386,34 @@ int launch_decode(DecodeArgs a, void* out, int64_t o_sb, int64_t o_sh, float* ls
   return launch_merge<T>(a, out, o_sb, o_sh, lse, st);
 }
 
+// Whether workgroup splits over 16-token pages are faster than one wave per split
+// with a page lookup per lane. A workgroup's start and the merge of its eight
+// waves have to pay for themselves: where a wave gets less than a step or two of
+// tokens (span), or many small workgroups queue for a CU, the small waves win.
+// Measured at 8 kv heads, one-wave splits / workgroup splits, us:
+//   * one split, at most a round of workgroups (no merge launch): always; D 128,
+//     32 sequences of 100 tokens 9.6 / 6.9;
+//   * one split, more rounds: D 128, 300 sequences of 100 tokens 25 / 49, of 400
+//     65 / 72, of 600 100 / 85; 128 sequences of 200 28 / 30, of 400 41 / 34; D 64
+//     (two workgroups a CU) 96 of 30 tokens 7.8 / 8.7, of 150 11.5 / 9.9, 500 of
+//     200 29 / 37, of 600 74 / 60. So 80 tokens a round, 48 at D 64, up to 512;
+//   * several splits: 1 sequence of 2000 (64 a split) 9.4 / 10.3, of 6000 (192)
+//     14.7 / 10.7; 8 of 600 (192) 8.1 / 8.4 at D 64, of 900 (256) 11.0 / 10.1 at
+//     D 128; two splits that leave CUs idle (12 sequences) at D 64, of 600 8.6 /
+//     9.8, of 1200 10.6 / 11.3, and about equal from 2000 on.
+// (choose_split_tokens, the caller's choice of split sizes, mirrors it.)
+bool half_page_splits_pay(int64_t units, int64_t span, int64_t max_splits, int64_t D,
+                          int64_t capacity) {
+  const int64_t cus = lc_cu_count();
+  if (max_splits == 1) {
+    const int64_t round = cus * (D <= 64 ? 2 : 1), rounds = (units + round - 1) / round;
+    const int64_t tokens = (D <= 64 ? 48 : 80) * rounds;
+    return rounds <= 1 || span >= (tokens < 512 ? tokens : 512);
+  }
+  return capacity >= 896 && span >= 192 &&
+         (max_splits > 2 || span >= 1024 || 8 * units * max_splits >= 7 * cus);
+}
+
 // Validates a decode call and launches it with the given workspace (the
 // caller's, or the device scratch of the allocation-free entry point).
 int paged_decode_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh,
@@ -1492,10 +1520,12 @@ int paged_decode_impl(const char* who, const void* q, int64_t q_sb, int64_t q_sh
   const int64_t span = max_splits == 1 ? max_pages_per_seq * page_size : split_tokens;
   const int64_t wave_tokens = ((span + kStep - 1) / kStep + waves - 1) / waves * kStep;
   const int64_t units = B * Hkv * ((Hq / Hkv + 15) / 16);
-  // Pages of 16 tokens run the workgroup splits too, unmasked, two
-  // page lookups a step: 34 us against 62 us for one wave per split with a
+  // Pages of 16 tokens run the workgroup splits too where they pay, unmasked,
+  // two page lookups a step: 34 us against 62 us for one wave per split with a
   // page lookup per lane (16 sequences of up to 4000 tokens, cold).
   const bool half_pages = page_size == kStep / 2 && a.bias == nullptr &&
+                          half_page_splits_pay(units, span, max_splits, D,
+                                               max_pages_per_seq * page_size) &&
                           ((page_size - 1) * kv_s_tok + D) * esz < (1LL << 31);
   const bool cluster = (row_pages || half_pages) &&
                        (max_splits == 1 || split_tokens >= 2048 || units * max_splits <= 512) &&

@@ -861,14 +861,28 @@ def single_split_fits(capacity_tokens: int, page_size: int, head_dim: int) -> bo
     return page_size % 32 == 0 and _wave_window_fits(capacity_tokens, page_size, head_dim)
 
 
+def _half_page_splits_pay(units: int, span: int, max_splits: int, head_dim: int,
+                          capacity_tokens: int, n_cus: int) -> bool:
+    """Whether workgroup splits over 16-token pages beat one wave per split (mirrors
+    half_page_splits_pay of the library, which holds the measurements)."""
+    if max_splits == 1:
+        per_cu, tokens = (2, 48) if head_dim <= 64 else (1, 80)
+        rounds = -(-units // (per_cu * n_cus))
+        return rounds <= 1 or span >= min(512, tokens * rounds)
+    return (capacity_tokens >= 896 and span >= 192
+            and (max_splits > 2 or span >= 1024 or 8 * units * max_splits >= 7 * n_cus))
+
+
 def takes_workgroup_splits(units: int, split_tokens: int, max_splits: int, page_size: int,
-                           head_dim: int, capacity_tokens: int) -> bool:
+                           head_dim: int, capacity_tokens: int, n_cus: int = 256) -> bool:
     """The library's choice between one workgroup per split and one wave per
     split (mirrors lc_paged_decode_fwd for unmasked calls): workgroups for a
     single split, splits of >= 2048 tokens, or grids of <= 512 splits, on pages
-    of 16 or a multiple of 32 tokens."""
+    of a multiple of 32 tokens, or of 16 where they pay."""
     span = capacity_tokens if max_splits == 1 else split_tokens
-    return ((page_size % 32 == 0 or page_size == 16) and _wave_window_fits(span, page_size, head_dim)
+    pays = page_size == 16 and _half_page_splits_pay(units, span, max_splits, head_dim,
+                                                     capacity_tokens, n_cus)
+    return ((page_size % 32 == 0 or pays) and _wave_window_fits(span, page_size, head_dim)
             and (max_splits == 1 or split_tokens >= 2048 or units * max_splits <= 512))
 
 
@@ -900,21 +914,29 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
         2's shape); one round of the CUs for fewer units, whatever the batch
         (16 sequences of 1-16K tokens, 128 units: 115.7 us at 8192 against
         127-133 us at 512-2048).
-    On pages of 16 tokens each rule takes more splits where a wave's share
-    would touch over 64 pages. Where the library would run such a split size
+    On pages of 16 tokens (a lookup per half step, against one per lane and no
+    prefetch for one-wave splits) each rule takes more splits where a wave's share
+    would touch over 64 pages, and three things differ: fewer units than CUs make
+    one round whatever the lengths (3 sequences of 6000 tokens at 8 kv heads: 17.4
+    us in one round, 25.1 as the 90% rule's 19 splits each); ragged batches of
+    over two rounds of units within 4096 tokens are not split (96 of up to 3000 at
+    D 64: 58 us, 76 at 2048-token splits, 70 in one-wave splits); ragged batches of
+    head_dims that the tiles pad (not 64 or 128) stay in one-wave splits (D 256, 2 kv
+    heads, 96 of up to 1200: 32 us, 44 in workgroups). Where the library would run such a split size
     with one wave per split instead (see takes_workgroup_splits), or on other
     page sizes, one-wave splits: 512 tokens, shrunk until there are >= 1024 of them.
     """
     units = batch * n_kv_heads * ((group + 15) // 16)
     if units == 0:  # an empty batch launches nothing; any valid split will do
         return max(64, -(-capacity_tokens // 64) * 64)
-    half_pages = page_size == 16 and not masked
+    half_pages = (page_size == 16 and not masked
+                  and (head_dim in (64, 128) or uniform_length is not None))
     if (page_size % 32 == 0 or half_pages) and capacity_tokens > 0:
         def fits(s: int) -> bool:  # (pages of 32 tokens up: as ever, checked at the end)
             return not half_pages or _wave_window_fits(
                 -(-(-(-capacity_tokens // s)) // 64) * 64, page_size, head_dim)
 
-        if uniform_length is not None:
+        if uniform_length is not None and not (half_pages and units < n_cus):
             length = max(1, min(int(uniform_length), capacity_tokens))
             s = 1
             while s < 64:
@@ -927,6 +949,8 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
             s = -(-6 * n_cus // units)
             while True:
                 split = max(2048, -(-(-(-capacity_tokens // s)) // 1024) * 1024)
+                if half_pages and units > 2 * n_cus and capacity_tokens <= 4096:
+                    s, split = 1, capacity_tokens
                 if s >= 64 or _wave_window_fits(split, page_size, head_dim):
                     break
                 s += 1
@@ -944,7 +968,7 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
             split = -(-capacity_tokens // 64) * 64
         max_splits = -(-capacity_tokens // split)
         if takes_workgroup_splits(units, split, max_splits, page_size, head_dim,
-                                  capacity_tokens):
+                                  capacity_tokens, n_cus):
             return split
 
     def n_splits(split: int) -> int:

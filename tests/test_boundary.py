@@ -212,6 +212,37 @@ def test_kv_cache_argument_checks():
         c.append(torch.zeros(3, 2, 11, 8), torch.zeros(3, 2, 11, 8))
 
 
+def test_split_heuristic_of_16_token_pages():
+    """Workgroup splits where they were measured faster, one-wave splits (as with
+    a mask) elsewhere."""
+    from llm_cuda.kernels._ops import choose_split_tokens, takes_workgroup_splits
+
+    def route(batch, tokens, length=None, hkv=8, d=128):
+        cap = -(-tokens // 16) * 16
+        split = choose_split_tokens(batch, hkv, 4, cap, 16, d, length)
+        n = -(-cap // split)
+        return takes_workgroup_splits(batch * hkv, split, n, 16, d, cap), n
+
+    # short contexts: a wave's share would be a step at most
+    for batch, tokens in ((1, 100), (3, 600), (1, 2000), (16, 600), (300, 100), (300, 400),
+                          (500, 300)):
+        assert not route(batch, tokens)[0] and not route(batch, tokens, tokens)[0]
+        cap = -(-tokens // 16) * 16
+        assert (choose_split_tokens(batch, 8, 4, cap, 16)
+                == choose_split_tokens(batch, 8, 4, cap, 16, masked=True))
+    # a single split of at most a round of workgroups, and of more with more tokens
+    for batch, tokens in ((32, 100), (64, 300), (128, 400), (300, 600)):
+        assert route(batch, tokens) == (True, 1) == route(batch, tokens, tokens)
+    assert route(64, 100, d=64) == (True, 1) and not route(96, 30, d=64)[0]
+    # one round of the CUs whatever the lengths
+    assert route(3, 6000, 6000) == route(3, 6000) == (True, 10)
+    assert route(1, 6000) == (True, 32) and route(16, 4000) == (True, 2)
+    # ragged batches of over two rounds of units: one split; fewer: the 2048-token floor
+    assert route(96, 3000, d=64) == (True, 1) and route(48, 3000) == (True, 2)
+    # head_dims that the tiles pad: workgroups for equal lengths only
+    assert not route(24, 3000, hkv=2, d=256)[0] and route(24, 3000, 3000, hkv=2, d=256)[0]
+
+
 def test_split_heuristic():
     from llm_cuda.kernels._ops import choose_split_tokens, takes_workgroup_splits
 

@@ -52,16 +52,22 @@ def _reference(q, kp, vp, bt, sl):
 
 @pytest.mark.parametrize("lens,Hq,Hkv,D,dtype,bad,split", [
     ([0, 1, 15, 16, 17, 31, 32, 33], 8, 2, 128, torch.bfloat16, (), None),
-    ([700, 513, 80], 8, 2, 64, torch.float16, ((0, 3), (0, 4), (1, 31)), None),
+    ([700, 513, 80], 8, 2, 64, torch.float16, ((0, 3), (0, 4), (1, 31)), 768),
+    ([1500, 1033, 80], 8, 2, 64, torch.float16, ((0, 3), (0, 40), (1, 64)), 192),
     ([2500] + [100 * i + 7 for i in range(39)], 32, 8, 128, torch.bfloat16, ((5, 0),), None),
-    ([300, 47], 40, 2, 256, torch.float16, (), None),   # two head groups
-    ([2047, 900], 4, 1, 96, torch.bfloat16, ((0, 127),), 128),
+    ([300, 47], 40, 2, 256, torch.float16, (), 320),   # two head groups
+    ([2047, 900], 4, 1, 96, torch.bfloat16, ((0, 127),), 256),
     ([7900, 60], 4, 2, 128, torch.bfloat16, (), 7936),  # the longest single split
 ])
 def test_page16_decode(cuda, lens, Hq, Hkv, D, dtype, bad, split):
     from llm_cuda.kernels.triton.decode_attention import paged_decode_attention
 
+    from llm_cuda.kernels import _ops
+
     args = _call(lens, Hq, Hkv, D, dtype, cuda, bad)
+    capacity, units = args[3].shape[1] * 16, len(lens) * Hkv * -(-(Hq // Hkv) // 16)
+    used = split or _ops.choose_split_tokens(len(lens), Hkv, Hq // Hkv, capacity, 16, D)
+    assert _ops.takes_workgroup_splits(units, used, -(-capacity // used), 16, D, capacity)
     out, lse = paged_decode_attention(*args, return_lse=True, split_tokens=split)
     ref, ref_lse = _reference(*args)
     assert (out.double() - ref).abs().max().item() <= ATOL[dtype]
