@@ -886,7 +886,6 @@ def takes_workgroup_splits(units: int, split_tokens: int, max_splits: int, page_
             and (max_splits == 1 or split_tokens >= 2048 or units * max_splits <= 512))
 
 
-@functools.lru_cache(maxsize=4096)
 def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens: int,
                         page_size: int = 64, head_dim: int = 128,
                         uniform_length: int | None = None, n_cus: int = 256,
@@ -926,6 +925,16 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
     with one wave per split instead (see takes_workgroup_splits), or on other
     page sizes, one-wave splits: 512 tokens, shrunk until there are >= 1024 of them.
     """
+    # (kept by value: what int() takes, a 0-d tensor for instance, may change in place)
+    return _choose_split_tokens(batch, n_kv_heads, group, capacity_tokens, page_size, head_dim,
+                                None if uniform_length is None else int(uniform_length), n_cus,
+                                masked)
+
+
+@functools.lru_cache(maxsize=4096)
+def _choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens: int,
+                         page_size: int, head_dim: int, uniform_length: int | None, n_cus: int,
+                         masked: bool) -> int:
     units = batch * n_kv_heads * ((group + 15) // 16)
     if units == 0:  # an empty batch launches nothing; any valid split will do
         return max(64, -(-capacity_tokens // 64) * 64)
@@ -937,7 +946,7 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
                 -(-(-(-capacity_tokens // s)) // 64) * 64, page_size, head_dim)
 
         if uniform_length is not None and not (half_pages and units < n_cus):
-            length = max(1, min(int(uniform_length), capacity_tokens))
+            length = max(1, min(uniform_length, capacity_tokens))
             s = 1
             while s < 64:
                 n = units * s

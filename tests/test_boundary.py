@@ -212,6 +212,17 @@ def test_kv_cache_argument_checks():
         c.append(torch.zeros(3, 2, 11, 8), torch.zeros(3, 2, 11, 8))
 
 
+def test_split_heuristic_follows_a_length_that_changes_in_place():
+    from llm_cuda.kernels._ops import choose_split_tokens
+
+    sizes = (8, 8, 4, 33024, 64, 128)
+    short, long = choose_split_tokens(*sizes, 2049), choose_split_tokens(*sizes, 32768)
+    length = torch.tensor(2049)
+    assert choose_split_tokens(*sizes, length) == short != long
+    length.fill_(32768)
+    assert choose_split_tokens(*sizes, length) == long
+
+
 def test_split_heuristic_of_16_token_pages():
     """Workgroup splits where they were measured faster, one-wave splits (as with
     a mask) elsewhere."""
