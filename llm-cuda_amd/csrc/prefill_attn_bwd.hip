@@ -507,8 +507,10 @@ attn_bwd_dkv_f32_kernel(BwdArgs a, int n_kb, int cus) {
     __builtin_amdgcn_sched_barrier(0);
     f32_dot_lds<DPAD>(dp, dor, v_lds + l32 * LD + hh * 4);
     lc_compiler_fence();
-    const bool edge = q0 + a.q_offset < key0 + kF32Rows - 1;
-    const int row_lim = kj - q0 - a.q_offset - 4 * hh;  // row c + 4hh sees the key from c = row_lim on
+    // Row c + 4hh sees the key from c = row_lim on, and is a row below row_end
+    // (past the end 0 * K is no 0 where K holds an inf or NaN).
+    const bool edge = q0 + a.q_offset < key0 + kF32Rows - 1 || q0 + kF32Rows > a.Sq;
+    const int row_lim = kj - q0 - a.q_offset - 4 * hh, row_end = a.Sq - q0 - 4 * hh;
     auto softmax_grad = [&](auto mask_c) __attribute__((always_inline)) {
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -518,10 +520,10 @@ attn_bwd_dkv_f32_kernel(BwdArgs a, int n_kb, int cus) {
         for (int i = 0; i < 4; ++i) {
           const int r = 4 * j + i, c = 8 * j + i;
           float x = s[r] * a.scale_log2 - l4[i];
-          bool masked = decltype(mask_c)::value && c < row_lim;
+          bool masked = decltype(mask_c)::value && (c < row_lim || c >= row_end);
           if constexpr (BIAS) {
             const int row = q0 + c + 4 * hh;
-            if (!masked && row < a.Sq && kj < a.Skv) {
+            if (!masked && kj < a.Skv) {
               const float bias = lc_bias_log2(lc_load_bias(
                   a.bias, b * a.bs[0] + h * a.bs[1] + (int64_t)row * a.bs[2] + (int64_t)kj * a.bs[3],
                   a.bias_dtype));

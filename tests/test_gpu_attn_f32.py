@@ -113,3 +113,22 @@ def test_f32_masked_pairs_touch_no_nonfinite_value(cuda, D, bad):
     ref = _run(q, k, v, do)
     for x, r in zip(got[3:], ref[3:]):  # keys after the bad queries: dk, dv
         assert (x[:, :, at:] - r[:, :, at:]).abs().max().item() <= bound
+
+
+@pytest.mark.parametrize("masked", [False, True])
+@pytest.mark.parametrize("S,Skv", [(50, 90), (33, 64), (1, 40)])
+@pytest.mark.parametrize("bad", [math.inf, math.nan])
+def test_f32_keys_that_no_query_sees(cuda, bad, S, Skv, masked):
+    """Infinite or NaN values of keys past every query's view (the unused end of a
+    buffer) in the query rows' last, partial tile: their gradients are zero, the
+    others those of the visible keys alone."""
+    bound = (32 + Skv) * 2.0 ** -23 * 8.0
+    q, k, v, do = _inputs(1, 2, 1, S, Skv, 32, cuda, seed=S)
+    mask = torch.zeros(1, 1, S, Skv, device=cuda) if masked else None
+    ref = _run(q, k[:, :, :S], v[:, :, :S], do)
+    k[:, :, S:] = bad
+    v[:, :, S:, 3] = bad
+    got = _run(q, k, v, do, mask=mask)
+    for x, r in zip(got, ref):
+        assert (x[:, :, :S] - r).abs().max().item() <= bound
+    assert all((x[:, :, S:] == 0).all() for x in got[3:])
