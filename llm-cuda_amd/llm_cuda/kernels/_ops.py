@@ -750,17 +750,34 @@ def _watched() -> bool:
             or torch.compiler.is_compiling())
 
 
+def _linear_f32_pays(M: int, N: int, K: int) -> bool:
+    """Where lc_linear_f32 is no slower than the library's GEMM even without the 11
+    us of host time that the library's call costs more eagerly (8.3 against 19.5):
+    at most 256 tiles of 32 x 32 (one round of the CUs; N 1376, K 256, 344 tiles 7.2
+    us here, 5.7 there) and
+
+      * K <= 256, which its eight waves contract in one step each;
+      * at most 256 rows and columns, where the library runs a few workgroups that
+        contract all of K; or
+      * K no multiple of 32, up to 512, or with over 65536 outputs (rows of whole
+        128-byte lines slow the operand loads by a quarter at K 640-768).
+
+    Graph-replayed us here / library: M 128, N 512, K 256 4.8 / 5.7, K 288 5.9 / 5.2,
+    K 300 5.3 / 5.9, K 496 5.5 / 7.1, K 512 6.5 / 6.4, K 640 8.2 / 5.2, K 688 6.9 /
+    6.1; M 512, N 512, K 688 7.0 / 7.7; M 128, N 256, K 688 6.9 / 83, K 768 8.9 / 88;
+    M 512, N 256, K 688 7.0 / 7.3, K 768 9.0 / 6.4. M <= 8 gives K 64 4.1 / 3.9 and
+    K 256 4.3 / 4.2 at N >= 384, otherwise at least the library's time within 3%."""
+    if not 0 < -(-M // 32) * -(-N // 32) <= 256 or K > 768:
+        return False
+    return (K <= 256 or (M <= 256 and N <= 256)
+            or (K % 32 != 0 and (K <= 512 or M * N > 65536)))
+
+
 def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
     """True where linear_f32 takes a projection over from the library's GEMM:
-    fp32 on the GPU, K <= 768, at most 256 tiles of 32 x 32 outputs, no autograd
-    graph being recorded, no autocast, plain tensors, nothing that follows
-    torch's calls (see _watched), and not inside torch_projections().
-
-    The line: one round of the CUs and a K that eight waves contract in a few
-    microseconds. Graph-replayed us a call, here / library: K 256, N 512, 64
-    tiles 4.5 / 5.7, 256 tiles 5.0 / 5.8, N 1376, 344 tiles 7.2 / 5.7; N 256, 64
-    tiles, K 688 6.7 / 160, K 1024 10.6 / 6.0; N 384, K 384 5.8 / 5.4 (the
-    library's call costs 13 us more on the host)."""
+    fp32 on the GPU, sizes where it pays (_linear_f32_pays), no autograd graph
+    being recorded, no autocast, plain tensors, nothing that follows torch's
+    calls (see _watched), and not inside torch_projections()."""
     if not _NATIVE_PROJECTIONS[0] or not (x.is_cuda and weight.is_cuda):
         return False
     if type(x) not in _PLAIN or type(weight) not in _PLAIN:  # (a subclass has its own linear)
@@ -768,10 +785,9 @@ def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
     if not (x.dtype == weight.dtype == torch.float32 and weight.dim() == 2 and x.dim() >= 1):
         return False
     N, K = weight.shape
-    if not (0 < K <= 768 and N > 0 and K % 4 == 0 and N % 4 == 0 and x.shape[-1] == K):
+    if not (K > 0 and N > 0 and K % 4 == 0 and N % 4 == 0 and x.shape[-1] == K):
         return False
-    rows = x.numel() // K
-    if not 0 < -(-rows // 32) * -(-N // 32) <= 256:
+    if not _linear_f32_pays(x.numel() // K, N, K):
         return False
     if _records_grad(x, weight) or torch.is_autocast_enabled() or _watched():
         return False

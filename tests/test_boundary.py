@@ -212,6 +212,21 @@ def test_kv_cache_argument_checks():
         c.append(torch.zeros(3, 2, 11, 8), torch.zeros(3, 2, 11, 8))
 
 
+def test_linear_f32_line():
+    """Sizes measured no slower than the library's GEMM under a graph, and those
+    measured slower."""
+    from llm_cuda.kernels._ops import _linear_f32_pays as pays
+
+    for M, N, K in ((1, 64, 64), (128, 512, 256), (256, 1024, 256), (128, 256, 688), (8, 256, 768),
+                    (256, 256, 512), (128, 512, 300), (8, 2048, 496), (512, 256, 688),
+                    (1024, 256, 688), (64, 1376, 688), (512, 512, 700)):
+        assert pays(M, N, K)
+    for M, N, K in ((0, 64, 64), (8, 1376, 384), (128, 384, 384), (512, 256, 512), (128, 512, 640),
+                    (8, 512, 688), (128, 512, 688), (512, 128, 688), (512, 256, 768),
+                    (64, 64, 772), (128, 2080, 256), (288, 1024, 256)):
+        assert not pays(M, N, K)
+
+
 def test_split_heuristic_follows_a_length_that_changes_in_place():
     from llm_cuda.kernels._ops import choose_split_tokens
 
