@@ -737,6 +737,10 @@ def decode_linear_partials(x: torch.Tensor, weight: torch.Tensor, shares: int = 
 # models/llama3/attention.py:100-102,154 and mlp.py:35-43)
 # ---------------------------------------------------------------------------
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+# (looked up once: these questions are asked on every small projection)
+_dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
+_functorch_level, _is_tracing = torch._C._functorch.maybe_current_level, torch._C._is_tracing
+_is_compiling = torch.compiler.is_compiling
 
 
 def _watched() -> bool:
@@ -744,10 +748,8 @@ def _watched() -> bool:
     native launch: a function or dispatch mode (FLOP counters, fake tensors), a
     functorch transform (vmap, jvp), a trace, or a forward-mode level, whose
     tangents F.linear carries."""
-    return (torch._C._len_torch_dispatch_stack() > 0 or torch._C._len_torch_function_stack() > 0
-            or torch._C._functorch.maybe_current_level() is not None
-            or _forward_ad._current_level >= 0 or torch._C._get_tracing_state() is not None
-            or torch.compiler.is_compiling())
+    return (_forward_ad._current_level >= 0 or _dispatch_modes() > 0 or _function_modes() > 0
+            or _functorch_level() is not None or _is_tracing() or _is_compiling())
 
 
 def _linear_f32_pays(M: int, N: int, K: int) -> bool:
@@ -802,6 +804,11 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
         raise TypeError("linear_f32 takes fp32 tensors")
     if weight.dim() != 2 or x.shape[-1] != weight.shape[1]:
         raise ValueError(f"x {tuple(x.shape)} and weight {tuple(weight.shape)} do not match")
+    return _linear_f32(x, weight)
+
+
+def _linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """linear_f32 of arguments that linear_f32_applies (or linear_f32) has looked at."""
     dev = nat.require_device(x, weight)
     N, K = weight.shape
     M = x.numel() // K if K else 0
@@ -825,31 +832,39 @@ def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 def linear(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     """x @ weight.T: linear_f32 where it applies, else F.linear."""
     if linear_f32_applies(x, weight):
-        return linear_f32(x, weight)
+        return _linear_f32(x, weight)
     return F.linear(x, weight)
 
 
-_LINEAR_FORWARD = torch.nn.Linear.forward
+_Linear, _LINEAR_FORWARD = torch.nn.Linear, torch.nn.Linear.forward
+# (the dicts themselves: hooks are entered into them)
+_FORWARD_HOOKS, _FORWARD_PRE_HOOKS, _BACKWARD_HOOKS, _BACKWARD_PRE_HOOKS = (
+    _module._global_forward_hooks, _module._global_forward_pre_hooks,
+    _module._global_backward_hooks, _module._global_backward_pre_hooks)
 
 
 def _is_plain_linear(module: torch.nn.Module) -> bool:
     """Whether module(x) is F.linear(x, module.weight) and nothing else: an
     nn.Linear itself without bias, hooks or a compiled call, whose forward nobody
     replaced (on the instance, as wrappers and quantisers do, or on the class)."""
-    return (type(module) is torch.nn.Linear and module.bias is None
-            and "forward" not in module.__dict__ and torch.nn.Linear.forward is _LINEAR_FORWARD
-            and module._compiled_call_impl is None
-            and not (module._forward_hooks or module._forward_pre_hooks
-                     or module._backward_hooks or module._backward_pre_hooks
-                     or _module._global_forward_hooks or _module._global_forward_pre_hooks
-                     or _module._global_backward_hooks or _module._global_backward_pre_hooks))
+    if type(module) is not _Linear or _Linear.forward is not _LINEAR_FORWARD:
+        return False
+    own = module.__dict__
+    return (own["_parameters"].get("bias") is None and "forward" not in own
+            and own.get("_compiled_call_impl") is None
+            and not (own["_forward_hooks"] or own["_forward_pre_hooks"]
+                     or own["_backward_hooks"] or own["_backward_pre_hooks"]
+                     or _FORWARD_HOOKS or _FORWARD_PRE_HOOKS
+                     or _BACKWARD_HOOKS or _BACKWARD_PRE_HOOKS))
 
 
 def project(x: torch.Tensor, module: torch.nn.Module) -> torch.Tensor:
     """module(x) for a projection; a plain nn.Linear (see _is_plain_linear) runs as
     linear_f32 where that applies."""
-    if _is_plain_linear(module) and linear_f32_applies(x, module.weight):
-        return linear_f32(x, module.weight)
+    if _is_plain_linear(module):
+        weight = module.weight
+        if linear_f32_applies(x, weight):
+            return _linear_f32(x, weight)
     return module(x)
 
 
