@@ -132,7 +132,8 @@ LC_API int lc_rope_fwd(const void* x1, void* out1, int64_t h1, const int64_t* x1
  * (fp32 or the dtype of q). Entries below -1e30 (and NaN) act as -1e30, so a
  * row whose visible keys are all so masked averages them, as the reference's
  * softmax of equal scores does; -inf excludes a key, and a row without any
- * visible key gives o = 0, lse = -inf (the reference gives NaN there).
+ * visible key gives o = 0, lse = -inf (the reference gives NaN there). The K
+ * and V rows of keys without weight may be left unread.
  * Hq % Hkv == 0. bf16/f16 (D a multiple of 8 up to 128) and fp32 (D a multiple
  * of 4 up to 128) run on MFMA; other cases run a generic fp32-FMA kernel
  * (D <= 256).

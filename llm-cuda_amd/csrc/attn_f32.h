@@ -14,10 +14,12 @@
 //     halves, so the accumulator is the B operand as it stands. Accumulator row
 //     i of d tile dt stands for dim DTL i + dt, so a lane reads its DTL dims of
 //     row n as one contiguous load (a wave: two whole rows).
-// Operands come straight from global memory (L2) into registers: an MFMA of
-// this type takes 64 cycles of its SIMD, so a tile's loads (16 row and 16
-// column instructions per 32 x 64 operand) are a small share of its time and
-// LDS staging, with its barriers, would buy nothing.
+// Streamed operands come straight from global memory (L2) into registers: an
+// MFMA of this type takes 64 cycles of its SIMD, so a tile's loads (16 row and 16
+// column instructions per 32 x 64 operand) are a small share of its time. What a
+// workgroup keeps is held in registers in the forward and dQ kernels and, where
+// those would cost the second wave (dK/dV: 182 against 95 us at [2, 16/8, 1024,
+// 64]), in LDS (f32_stage).
 #pragma once
 
 #include "attn_tiles.h"

@@ -45,6 +45,8 @@ def _reference(q, k, v, mask, off):
 @pytest.mark.parametrize("Sq,Skv,D,dtype,mdt", [
     (200, 200, 128, torch.bfloat16, torch.bfloat16),
     (77, 133, 64, torch.float16, torch.float32),
+    (2, 65, 128, torch.bfloat16, torch.float32),
+    # one query row: expand keeps its stride, so the row-bias kernel on both sides
     (1, 65, 128, torch.bfloat16, torch.float32),
 ])
 def test_key_mask(cuda, kind, Sq, Skv, D, dtype, mdt):
@@ -124,19 +126,18 @@ def test_key_mask_at_the_most_keys_staged(cuda, Skv):
     assert (out.double() - ref).abs().max().item() <= ATOL[dtype]
 
 
-@pytest.mark.parametrize("value", ["min", -1e9, -1e20])
-@pytest.mark.parametrize("D,dtype", [(40, torch.bfloat16), (56, torch.bfloat16),
-                                     (64, torch.float16), (104, torch.bfloat16),
-                                     (112, torch.float16), (128, torch.bfloat16),
-                                     (64, torch.float32)])
+@pytest.mark.parametrize("value,D,dtype", [
+    (value, D, dtype) for value in ("min", -1e9, -1e20)
+    for D, dtype in ((40, torch.bfloat16), (56, torch.bfloat16), (64, torch.float16),
+                     (104, torch.bfloat16), (112, torch.float16), (128, torch.bfloat16),
+                     (64, torch.float32))
+    if value != -1e20 or dtype != torch.float16])  # (-1e20: not a float16 value)
 def test_left_padded_gradients(cuda, value, D, dtype):
     """A training step over a left-padded batch, no gradient arriving at the pad
     rows (all of whose keys are masked): the gradients are those of the prompts
     alone, zero at the pads, and those of the mask written out per row."""
     from llm_cuda.kernels.triton.attention import triton_fused_causal_attention
 
-    if value == -1e20 and dtype == torch.float16:
-        pytest.skip("not a float16 value")
     B, Hq, Hkv, S, pads = 2, 4, 2, 150, (90, 0)
     g = torch.Generator().manual_seed(D)
     mdt = torch.float32 if dtype == torch.float16 and value == -1e9 else dtype
