@@ -737,6 +737,7 @@ def decode_linear_partials(x: torch.Tensor, weight: torch.Tensor, shares: int = 
 # models/llama3/attention.py:100-102,154 and mlp.py:35-43)
 # ---------------------------------------------------------------------------
 _PLAIN = (torch.Tensor, torch.nn.Parameter)
+_STRIDED = torch.strided
 # (looked up once: these questions are asked on every small projection)
 _dispatch_modes, _function_modes = torch._C._len_torch_dispatch_stack, torch._C._len_torch_function_stack
 _functorch_level, _is_tracing = torch._C._functorch.maybe_current_level, torch._C._is_tracing
@@ -784,6 +785,8 @@ def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
         return False
     if type(x) not in _PLAIN or type(weight) not in _PLAIN:  # (a subclass has its own linear)
         return False
+    if x.layout is not _STRIDED or weight.layout is not _STRIDED:  # (sparse: no rows to read)
+        return False
     if not (x.dtype == weight.dtype == torch.float32 and weight.dim() == 2 and x.dim() >= 1):
         return False
     N, K = weight.shape
@@ -793,7 +796,8 @@ def linear_f32_applies(x: torch.Tensor, weight: torch.Tensor) -> bool:
         return False
     if _records_grad(x, weight) or torch.is_autocast_enabled() or _watched():
         return False
-    return weight.stride(1) == 1 and (N == 1 or K <= weight.stride(0) < 2 ** 23)
+    row, col = weight.stride()
+    return col == 1 and (N == 1 or K <= row < 2 ** 23)
 
 
 def linear_f32(x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:

@@ -100,3 +100,17 @@ def test_linear_stays_with_torch_where_its_calls_are_followed(cuda):
     traced = torch.jit.trace(lambda u: _ops.linear(u, w), x)
     assert torch.allclose(traced(3 * x), F.linear(3 * x, w), atol=1e-4)
     assert _ops.linear_f32_applies(x, w)
+
+
+def test_project_of_a_sparse_weight(cuda):
+    """A pruned weight, which F.linear takes (CSR has no strides to ask for)."""
+    from llm_cuda.kernels import _ops
+
+    g = torch.Generator().manual_seed(3)
+    x, w = torch.randn(4, 64, generator=g).to(cuda), torch.randn(32, 64, generator=g).to(cuda)
+    for sparse in (w.to_sparse_csr(), w.to_sparse()):
+        lin = torch.nn.Linear(64, 32, bias=False, device=cuda)
+        lin.weight = torch.nn.Parameter(sparse, requires_grad=False)
+        assert not _ops.linear_f32_applies(x, lin.weight)
+        assert torch.equal(_ops.project(x, lin), F.linear(x, sparse))
+    assert not _ops.linear_f32_applies(x.to_sparse_csr(), w)
