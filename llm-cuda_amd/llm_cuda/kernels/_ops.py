@@ -854,7 +854,8 @@ def _is_plain_linear(module: torch.nn.Module) -> bool:
     if type(module) is not _Linear or _Linear.forward is not _LINEAR_FORWARD:
         return False
     own = module.__dict__
-    return (own["_parameters"].get("bias") is None and "forward" not in own
+    # (a bias that is no parameter, as in a DataParallel replica, is not found there)
+    return (own["_parameters"].get("bias", own) is None and "forward" not in own
             and own.get("_compiled_call_impl") is None
             and not (own["_forward_hooks"] or own["_forward_pre_hooks"]
                      or own["_backward_hooks"] or own["_backward_pre_hooks"]

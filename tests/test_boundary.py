@@ -227,6 +227,26 @@ def test_linear_f32_line():
         assert not pays(M, N, K)
 
 
+def test_a_bias_outside_the_parameters_is_a_bias():
+    """As a plain tensor (a DataParallel replica's) or a buffer."""
+    from llm_cuda.kernels._ops import _is_plain_linear
+
+    def linear(bias):
+        return torch.nn.Linear(8, 4, bias=bias)
+
+    assert _is_plain_linear(linear(False)) and not _is_plain_linear(linear(True))
+    replica = linear(True)._replicate_for_data_parallel()
+    replica.weight, replica.bias = torch.zeros(4, 8), torch.ones(4)
+    assert "bias" not in replica._parameters and not _is_plain_linear(replica)
+    buffered = linear(True)
+    del buffered.bias
+    buffered.register_buffer("bias", torch.ones(4))
+    assert not _is_plain_linear(buffered)
+    removed = linear(True)
+    removed.bias = None
+    assert _is_plain_linear(removed)
+
+
 def test_split_heuristic_follows_a_length_that_changes_in_place():
     from llm_cuda.kernels._ops import choose_split_tokens
 
