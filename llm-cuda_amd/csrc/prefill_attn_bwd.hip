@@ -24,6 +24,7 @@
 //   * everything else: lane-per-row fp32 kernels.
 #include <math.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "attn_f32.h"
@@ -958,6 +959,10 @@ __device__ __host__ __forceinline__ int dkv_tiles(int kb, int n_qt, int q_offset
 __device__ __host__ __forceinline__ int dkv_shares(int tiles, int share) {
   return tiles <= share ? 1 : (tiles + share - 1) / share;
 }
+// First tile of the i-th of a block's shares (even: a share starts in buffer 0).
+__device__ __host__ __forceinline__ int dkv_share_begin(int tiles, int i, int shares) {
+  return i == shares ? tiles : static_cast<int>((int64_t)tiles * i / shares) & ~1;
+}
 
 // SPLIT: a causal grid of few key blocks ends with its first block, whose tiles
 // are twice the mean, and a short one leaves most CUs without a block: the
@@ -1277,11 +1282,11 @@ attn_bwd_dkv_mfma_kernel(BwdArgs a) {
     }
   };
 
-  // This workgroup's iterations (a share starts on an even one: buffer 0).
+  // This workgroup's iterations.
   int it0 = 0, it1 = n_iter;
   if constexpr (SPLIT) {
-    it0 = static_cast<int>((int64_t)n_iter * share / shares) & ~1;
-    it1 = share + 1 == shares ? n_iter : static_cast<int>((int64_t)n_iter * (share + 1) / shares) & ~1;
+    it0 = dkv_share_begin(n_iter, share, shares);
+    it1 = dkv_share_begin(n_iter, share + 1, shares);
   }
   // MASK: false / true for tiles known to be unmasked / on the diagonal,
   // kRuntimeMask to pick per tile (the bias path).
@@ -1388,15 +1393,64 @@ __global__ __launch_bounds__(256) void dkv_reduce_kernel(BwdArgs a) {
   }
 }
 
+// When a dK/dV grid ends, in tiles: its workgroups, one to a CU, go in order to
+// the CU that is free first; each costs its tiles and 2 more (start and stores).
+class DkvEnd {
+ public:
+  DkvEnd() : idle_(std::min(lc_cu_count(), kMaxCus)) {}
+  void add(int tiles, int64_t n) {  // n workgroups
+    if (tiles == 0) return;
+    while (n > 0) {
+      Cus c{0, idle_};
+      if (idle_ > 0) {
+        idle_ = 0;
+      } else {
+        std::pop_heap(heap_, heap_ + size_, later);
+        c = heap_[--size_];
+      }
+      const int take = static_cast<int>(std::min<int64_t>(n, c.count));
+      if (c.count > take && c.time == 0)
+        idle_ = c.count - take;
+      else if (c.count > take)
+        push({c.time, c.count - take});
+      push({c.time + tiles + 2, take});
+      end_ = std::max(end_, c.time + tiles + 2);
+      n -= take;
+    }
+  }
+  int64_t end() const { return end_; }
+
+ private:
+  static constexpr int kMaxCus = 1024;
+  struct Cus {  // CUs that are free from the same time on
+    int64_t time;
+    int count;
+  };
+  static bool later(const Cus& a, const Cus& b) { return a.time > b.time; }
+  void push(Cus c) {
+    heap_[size_++] = c;
+    std::push_heap(heap_, heap_ + size_, later);
+  }
+  Cus heap_[kMaxCus];  // (each entry has a CU at least)
+  int size_ = 0, idle_;
+  int64_t end_ = 0;
+};
+
 // How an unmasked MFMA call's dK/dV grid is dealt out (share 0: one workgroup
 // per key block). A workgroup has a CU to itself, so a grid takes as long as its
 // first block unless the blocks fill several rounds: where that block has over
 // 1.4 times a CU's mean share of all tiles, blocks are dealt out in shares of 1.3
 // times the mean (at the mean itself a second round of small shares starts; the
-// fp32 sums and their launch cost more at smaller ones). us a backward, whole
+// fp32 sums and their launch cost more at smaller ones), provided that this grid
+// ends earlier by more than the sums cost: 5 tiles for the launch and 3 for each
+// round of the CUs that leaves sums. (Equal blocks, of a chunk over a long cached
+// prefix above all, may cut into two rounds of halves.) us a backward, whole
 // blocks / 1.0 / 1.3 / 1.6 of the mean, D 128, 32/8 heads: [1, 512] 85 / 57 /
 // 57 / 56, [1, 1024] 152 / 100 / 82 / 83, [1, 2048] 295 / 208 / 172 / 181,
-// [2, 2048] 337 / 315 / 294 / 308.
+// [2, 2048] 337 / 315 / 294 / 308. Whole blocks / shares of 1.3, of 700 sizes
+// with such a first block: 3 of those left in shares are slower (by 2%), 63 were
+// (by up to 33%: 78 queries over 886 keys, 3 sequences of 64/8 heads, 75.8 / 91.7;
+// 216 over 346, 8 of 32/8, 67.6 / 89.7); 10 of those left whole would gain, up to 5%.
 struct DkvPlan {
   int share;     // tiles per share
   int items;     // share items of a unit
@@ -1415,15 +1469,21 @@ DkvPlan dkv_plan(int64_t units, int64_t Sq, int64_t Skv, int64_t q_offset, int G
   const int64_t share = (mean * 13 + 9) / 10;
   if (most <= 2 * kDkvMinShare || most * 5 <= mean * 7) return p;
   p.share = static_cast<int>(share > kDkvMinShare ? share : kDkvMinShare);
+  DkvEnd whole, dealt;
   for (int kb = 0; kb < n_kb; ++kb) {
-    const int s = dkv_shares(dkv_tiles(kb, n_qt, (int)q_offset, G), p.share);
+    const int tiles = dkv_tiles(kb, n_qt, (int)q_offset, G);
+    const int s = dkv_shares(tiles, p.share);
     p.items += s;
+    whole.add(tiles, units);
+    for (int i = 0; i < s; ++i)
+      dealt.add(dkv_share_begin(tiles, i + 1, s) - dkv_share_begin(tiles, i, s), units);
     if (s > 1) {
       p.multi += s;
       ++p.blocks;
     }
   }
-  return p;
+  const int64_t cost = 5 + 3 * units * p.multi / lc_cu_count();
+  return whole.end() - dealt.end() > cost ? p : DkvPlan{0, 0, 0, 0};
 }
 int64_t dkv_part_bytes(const DkvPlan& p, int64_t units, int64_t D) {
   return p.share == 0 ? 0 : units * p.multi * (2LL * kBkKeys * (D <= 64 ? 64 : 128) * 4);

@@ -247,6 +247,23 @@ def test_a_bias_outside_the_parameters_is_a_bias():
     assert _is_plain_linear(removed)
 
 
+def test_dkv_shares_only_where_the_grid_ends_earlier():
+    """Backward sizes measured faster in shares of the dK/dV key blocks, and those
+    that would cut into more rounds of the CUs."""
+    from llm_cuda import _native as nat
+
+    def shared(B, Hq, Hkv, Sq, prefix, D):
+        return nat.load().lc_prefill_attn_bwd_split_bytes(
+            B, Hq, Hkv, Sq, Sq + prefix, D, prefix, 0, nat.DTYPE_BF16) > 0
+
+    for sizes in ((1, 32, 8, 512, 0, 128), (1, 32, 8, 2048, 0, 128), (2, 32, 8, 2048, 0, 128),
+                  (1, 32, 8, 1024, 0, 128), (2, 8, 2, 333, 267, 128)):
+        assert shared(*sizes)
+    for sizes in ((3, 64, 8, 78, 808, 128), (8, 32, 8, 216, 130, 128), (12, 32, 8, 141, 37, 128),
+                  (2, 28, 4, 1740, 1732, 128), (3, 16, 8, 313, 352, 64), (4, 32, 8, 4096, 0, 128)):
+        assert not shared(*sizes)
+
+
 def test_split_heuristic_follows_a_length_that_changes_in_place():
     from llm_cuda.kernels._ops import choose_split_tokens
 
