@@ -64,26 +64,60 @@ __device__ __forceinline__ void pf_barrier() {
 // unit about 5% more work than the fourth); alternating the direction gives
 // the four engines equal sums. A final partial run stays a permutation of
 // itself.
-__device__ __forceinline__ int pf_snake(int q, int n) {
+__device__ __host__ __forceinline__ int pf_snake(int q, int n) {
   const int s = (q & ~3) | ((q & 4) ? 3 - (q & 3) : (q & 3));
   return s < n ? s : q;
 }
 
-// Position of the q-th workgroup of an XCD in its heaviest-first list of n, for
-// a grid of more than one and at most two workgroups per CU, all of which start
-// at once: the ones that join a CU's first (from the pair_from-th on) run through
-// the rest of the list from its light end, so that a CU's two weigh about the
-// same. In list order the first CU gets the heaviest and the median one, 1.5
-// times the mean. Forward at 32/8 heads, D 128: [2, 1024] 36.6 -> 30.5 us, [4, 512]
-// 24.8 -> 22.0, [1, 2048] 47.9 -> 46.3; at 16/8, D 64: [2, 2048] 37.9 -> 31.1.
+// Position of the q-th workgroup of an XCD in its list of n (unit after unit,
+// heaviest first), for a grid of more than one and at most two workgroups per CU,
+// all of which start at once: the ones that join a CU's first (from the
+// pair_from-th on) run through the rest of the list from its end, so that a CU's
+// two weigh about the same. In list order, with one or two units to an XCD, the
+// first CU gets the heaviest and the median one, 1.5 times the mean. Forward at
+// 32/8 heads, D 128: [2, 1024] 36.6 -> 30.5 us, [4, 512] 24.8 -> 22.0, [1, 2048]
+// 47.9 -> 46.3; at 16/8, D 64: [2, 2048] 37.9 -> 31.1.
 __device__ __forceinline__ int pf_pair(int q, int n, int pair_from) {
   return q < pair_from ? q : n - 1 - (q - pair_from);
 }
-// pair_from for a grid of nwg workgroups (a list order that suits any other
-// grid: none reversed).
+// pair_from for any grid of nwg workgroups that starts at once (else: none).
+constexpr int kPfNoPairs = 0x7fffffff, kPfMostPaired = 1024;
 inline int pf_pair_from(int64_t nwg) {
   const int cus = lc_cu_count();
-  return nwg % 8 == 0 && nwg > cus && nwg <= 2LL * cus ? cus / 8 : 0x7fffffff;
+  return nwg % 8 == 0 && nwg > cus && nwg <= 2LL * cus && nwg <= kPfMostPaired ? cus / 8
+                                                                                : kPfNoPairs;
+}
+// pair_from of a causal grid, units of n_rbg row groups of `rows` query rows.
+// Pairs where the heaviest CU's two then hold over a tile of 64 keys less; with
+// many units to an XCD the list's end may be as heavy as the middle that it
+// replaces, and units of under 7 groups weigh too little for their tiles to tell
+// the times. Of 350 sizes 43 are slower by 2-8% if always paired (28/4 heads, [8,
+// 199] 15.0 / 16.4 us, [3, 748] 28.7 / 30.5), none so (of 400 others one by 3%),
+// and 45 left unpaired would gain, most of them 2-6%.
+inline int pf_pair_from(int64_t nwg, int n_rbg, int rows, int64_t Sq, int64_t Skv,
+                        int64_t q_offset) {
+  const int first = pf_pair_from(nwg);
+  if (first == kPfNoPairs || n_rbg < 7) return kPfNoPairs;
+  int tiles[kPfMostPaired];  // of a unit's workgroups in list order
+  for (int i = 0; i < n_rbg; ++i) {
+    const int64_t end = (int64_t)(n_rbg - pf_snake(i, n_rbg)) * rows;
+    const int64_t keys = (end < Sq ? end : Sq) + q_offset;
+    tiles[i] = static_cast<int>(((keys < Skv ? keys : Skv) + 63) / 64);
+  }
+  const int n = static_cast<int>(nwg / 8);
+  int list = 0, paired = 0;  // the heaviest CU's tiles
+  for (int x = 0, start = 0; x < 8; ++x, start = (start + n) % n_rbg) {
+    if (x > 0 && start == 0) break;  // (the XCDs from here on repeat the first ones)
+    for (int q = 0; q < first; ++q) {
+      const int w = tiles[(start + q) % n_rbg];
+      const bool two = first + q < n;
+      const int l = two ? w + tiles[(start + first + q) % n_rbg] : w;
+      const int p = two ? w + tiles[(start + n - 1 - q) % n_rbg] : w;
+      list = l > list ? l : list;
+      paired = p > paired ? p : paired;
+    }
+  }
+  return list - paired > 1 ? first : kPfNoPairs;
 }
 
 template <int CPR>

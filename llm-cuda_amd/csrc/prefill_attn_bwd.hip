@@ -1532,7 +1532,9 @@ int launch_bwd_mfma(BwdArgs a, int64_t part_bytes, hipStream_t st) {
   const int64_t nwg_k = (int64_t)n_kb * a.Hkv * a.B;
   LC_REQUIRE(nwg_q < (1LL << 31) && nwg_k < (1LL << 31), "lc_prefill_attn_bwd: grid too large");
   const int bias = a.bias == nullptr ? 0 : (a.bias_dtype == LC_DTYPE_F32 ? 2 : 1);
-  a.pair_from = bias == 0 ? pf_pair_from(nwg_q) : 0x7fffffff;  // (masked: one a CU)
+  // (masked: one a CU)
+  a.pair_from =
+      bias == 0 ? pf_pair_from(nwg_q, n_rbg, rbw * kBwRows, a.Sq, a.Skv, a.q_offset) : kPfNoPairs;
   if (nwg_q > 0) {
     if (bias == 0)
       launch_dq_mfma<T, 0>(a, (unsigned)nwg_q, hw, n_rbg, st);

@@ -210,3 +210,34 @@ def test_dynamic_tail_matches_static_order(cuda, B, Hq, Hkv, Sq, Skv, D):
                                         vc[:, :, :off + i + 1], q_offset=off + i)
         assert_close(ref_o[:, :, i:i + 1], o_ref, ATOL[torch.bfloat16], f"row {i}")
         assert_lse_close(ref_lse[:, :, i:i + 1], l_ref)
+
+
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,off,D", [
+    (2, 32, 8, 1000, 0, 128),  # two workgroups a CU, paired: whole units to an XCD
+    (2, 16, 8, 1628, 0, 64),   # XCDs that start inside a unit
+    (3, 28, 4, 740, 0, 128),   # short units, in list order
+    (4, 16, 16, 534, 100, 128),
+])
+@pytest.mark.parametrize("key_mask", [False, True])
+def test_grids_that_start_at_once(cuda, B, Hq, Hkv, Sq, off, D, key_mask):
+    """The order of the workgroups changes no result: each sequence as it comes out
+    alone, from a grid of at most one workgroup a CU."""
+    from llm_cuda.kernels import _ops
+
+    q, k, v = _qkv(B, Hq, Hkv, Sq, Sq + off, D, torch.bfloat16, cuda, seed=Sq)
+    do = torch.randn(q.shape, generator=torch.Generator().manual_seed(1)).to(q)
+    mask = None
+    if key_mask:
+        mask = torch.zeros(B, 1, 1, Sq + off, device=cuda)
+        for b in range(B):
+            mask[b, ..., :b * Sq // (2 * B)] = torch.finfo(torch.bfloat16).min
+
+    def run(rows):
+        m = None if mask is None else mask[rows]
+        out, lse = _ops.prefill_attention(q[rows], k[rows], v[rows], off, return_lse=True,
+                                          attention_mask=m)
+        return out, lse, _ops.prefill_attention_backward(
+            q[rows], k[rows], v[rows], out, lse, do[rows], off, attention_mask=m)[0]
+
+    for x, *alone in zip(run(slice(0, B)), *(run(slice(b, b + 1)) for b in range(B))):
+        assert torch.equal(x, torch.cat(alone))
