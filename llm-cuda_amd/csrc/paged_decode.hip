@@ -59,6 +59,9 @@ struct DecodeArgs {
   // workgroups below this block id always keep their id as rank.
   int* ord_ticket;
   int ord_static;
+  // Not 0: every sequence is cut into max_splits equal parts of its own length,
+  // of at least this many tokens (see split_tokens_of).
+  int own_split;
 };
 
 // Bias of token tok for (b, h), in the exp2 domain; 0 past bias_len.
@@ -66,6 +69,16 @@ __device__ __forceinline__ float decode_bias(const DecodeArgs& a, int b, int h, 
   return tok < a.bias_len
              ? lc_bias_log2(lc_load_bias(a.bias, b * a.bias_sb + h * a.bias_sh + tok, a.bias_dtype))
              : 0.f;
+}
+
+// Tokens per split of a sequence of len tokens: split_tokens (what the capacity
+// of the table gives), or with own_split an equal part of len, so that a sequence
+// far shorter than the table still has all of its workgroups (no more than
+// split_tokens, or own_split where that is more: split_tokens is a multiple of 64
+// and max_splits of them cover every len).
+__device__ __forceinline__ int split_tokens_of(const DecodeArgs& a, int len) {
+  if (a.own_split == 0) return a.split_tokens;
+  return max(a.own_split, ((len + a.max_splits - 1) / a.max_splits + 63) & ~63);
 }
 
 __device__ __forceinline__ int seq_len_of(const DecodeArgs& a, int b) {
@@ -749,7 +762,9 @@ __global__ __launch_bounds__(64 * cluster_waves<DPAD>()) void paged_decode_clust
   }
   const int cap = a.max_pages * a.P;
   // This workgroup's split: tokens [s_begin, s_begin + split_tokens).
-  const int s_begin = split * a.split_tokens;
+  constexpr bool OWN = P16 && !ORD;
+  const int split_tokens = OWN ? split_tokens_of(a, seq_len_of(a, b)) : a.split_tokens;
+  const int s_begin = split * split_tokens;
   // PRE (the split's pages fit 64 block-table entries): the window of the row
   // from the split's first page is loaded whole (one entry per lane) together
   // with the length, so the first K/V loads wait on one round trip, not on
@@ -771,7 +786,7 @@ __global__ __launch_bounds__(64 * cluster_waves<DPAD>()) void paged_decode_clust
   if (a.max_splits > 1 && s_begin >= len) return;
   const int prow = p_new < 0 ? 0 : min(p_new, sa.table_rows - 1);
   const int half = a.D / 2;
-  const int s_len = min(len - s_begin, a.split_tokens);
+  const int s_len = min(len - s_begin, split_tokens);
   const int nsteps = s_len > 0 ? (s_len + kStep - 1) / kStep : 0;
   const int t_begin = s_begin + (wave * nsteps / W) * kStep;
   const int t_end = min(len, s_begin + ((wave + 1) * nsteps / W) * kStep);
@@ -1178,7 +1193,8 @@ __global__ __launch_bounds__(64) void decode_merge_kernel(DecodeArgs a, T* __res
   const int h = blockIdx.x;
   const int b = blockIdx.y;
   const int len = seq_len_of(a, b);
-  const int nsplit = (len + a.split_tokens - 1) / a.split_tokens;
+  const int split_tokens = split_tokens_of(a, len);
+  const int nsplit = (len + split_tokens - 1) / split_tokens;
   const int64_t pbase = ((int64_t)b * a.Hq + h) * a.max_splits;
   T* oh = out + (int64_t)b * o_sb + (int64_t)h * o_sh;
   const int d0 = lane * VPL;
@@ -1271,7 +1287,7 @@ int launch_merge(const DecodeArgs& a, void* out, int64_t o_sb, int64_t o_sh, flo
 }
 
 template <typename T, int DPAD>
-int launch_cluster(const DecodeArgs& a, void* out, int64_t o_sb, int64_t o_sh, float* lse,
+int launch_cluster(DecodeArgs a, void* out, int64_t o_sb, int64_t o_sh, float* lse,
                    hipStream_t st) {
   // Split-major order (blockIdx.z = split), as in the one-wave kernel.
   dim3 grid(a.Hkv * a.n_hgroups, a.B, a.max_splits);
@@ -1305,10 +1321,12 @@ int launch_cluster(const DecodeArgs& a, void* out, int64_t o_sb, int64_t o_sh, f
     else
       paged_decode_cluster_kernel<T, DPAD, false, false, false, true>
           <<<g1, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
-  } else if (a.P % kStep != 0)
+  } else if (a.P % kStep != 0) {
+    // One round of workgroups: a step for each of a workgroup's waves at least.
+    if (a.max_splits > 1) a.own_split = cluster_waves<DPAD>() * kStep;
     paged_decode_cluster_kernel<T, DPAD, false, false, false, false, true>
         <<<grid, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
-  else if (a.bias != nullptr && pre)
+  } else if (a.bias != nullptr && pre)
     paged_decode_cluster_kernel<T, DPAD, true, false, true>
         <<<grid, threads, 0, st>>>(a, o, o_sb, o_sh, lse, none);
   else if (a.bias != nullptr)

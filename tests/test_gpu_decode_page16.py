@@ -79,3 +79,31 @@ def test_page16_decode(cuda, lens, Hq, Hkv, D, dtype, bad, split):
     lanes, llse = paged_decode_attention(*args, return_lse=True, attention_mask=zero)
     assert (out.float() - lanes.float()).abs().max().item() <= ATOL[dtype]
     assert (lse - llse)[live].abs().max().item() <= max(lens) * 2.0 ** -23 + 1e-5
+
+
+@pytest.mark.parametrize("lens,columns,split,Hq,Hkv,D,dtype", [
+    ([900, 1, 0, 255], 600, 320, 8, 2, 128, torch.bfloat16),      # parts of a step a wave
+    ([257, 512, 2049, 4097], 2000, 2048, 16, 4, 64, torch.float16),  # one token into another part
+    ([3000], 1875, 1024, 4, 1, 256, torch.bfloat16),
+    ([1700, 33] * 20, 520, 2816, 8, 2, 96, torch.float16),
+])
+def test_page16_short_sequences_in_a_wide_table(cuda, lens, columns, split, Hq, Hkv, D,
+                                                    dtype):
+    """Each sequence is cut by its own length, whatever the table's capacity: as in
+    a table of just its pages."""
+    from llm_cuda.kernels import _ops
+    from llm_cuda.kernels.triton.decode_attention import paged_decode_attention
+
+    q, kp, vp, bt, sl = args = _call(lens, Hq, Hkv, D, dtype, cuda)
+    wide = torch.full((len(lens), columns), -1, dtype=torch.int32, device=cuda)
+    wide[:, :bt.shape[1]] = bt
+    units, capacity = len(lens) * Hkv, columns * 16
+    n = -(-capacity // split)
+    assert n > 1 and units * n <= 256
+    assert _ops.takes_workgroup_splits(units, split, n, 16, D, capacity)
+    out, lse = paged_decode_attention(q, kp, vp, wide, sl, return_lse=True, split_tokens=split)
+    ref, ref_lse = _reference(*args)
+    assert (out.double() - ref).abs().max().item() <= ATOL[dtype]
+    live = torch.isfinite(ref_lse)
+    assert torch.equal(torch.isfinite(lse), live)
+    assert (lse.double() - ref_lse)[live].abs().max().item() <= max(lens) * 2.0 ** -24 + 1e-5
