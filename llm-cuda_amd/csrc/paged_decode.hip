@@ -1411,24 +1411,27 @@ int launch_decode(DecodeArgs a, void* out, int64_t o_sb, int64_t o_sh, float* ls
 // Measured at 8 kv heads, one-wave splits / workgroup splits, us:
 //   * one split, at most a round of workgroups (no merge launch): always; D 128,
 //     32 sequences of 100 tokens 9.6 / 6.9;
-//   * one split, more rounds: D 128, 300 sequences of 100 tokens 25 / 49, of 400
-//     65 / 72, of 600 100 / 85; 128 sequences of 200 28 / 30, of 400 41 / 34; D 64
-//     (two workgroups a CU) 96 of 30 tokens 7.8 / 8.7, of 150 11.5 / 9.9, 500 of
-//     200 29 / 37, of 600 74 / 60. So 80 tokens a round, 48 at D 64, up to 512;
-//   * several splits: 1 sequence of 2000 (64 a split) 9.4 / 10.3, of 6000 (192)
-//     14.7 / 10.7; 8 of 600 (192) 8.1 / 8.4 at D 64, of 900 (256) 11.0 / 10.1 at
-//     D 128; two splits that leave CUs idle (12 sequences) at D 64, of 600 8.6 /
-//     9.8, of 1200 10.6 / 11.3, and about equal from 2000 on.
+//   * one split, two or three rounds: from 80 tokens of capacity a round, 48 at D 64
+//     (two workgroups a CU; 96 sequences of 30 tokens 7.8 / 8.7, of 150 11.5 / 9.9),
+//     1.3 times as fast on full tables, 1.2 on ones filled to 12-50%; emptier ones
+//     0.8 (76 of up to 23 in 457: 10.2 / 15.7);
+//   * one split, more rounds: never. Every workgroup's start counts where contexts
+//     are short: 1.2 times as fast on full tables, but 0.6 on ones filled to under
+//     12% (258 sequences of up to 34 in 1061, 16 kv heads: 18.5 / 75; 270 of up to
+//     278 in 1232: 45 / 57);
+//   * several splits: from 1792 tokens of capacity. Below, 1.04 to 1.06 times as fast
+//     on full tables, 0.9 on emptier ones (9 of up to 995 at D 64: 9.3 / 10.6); 1
+//     sequence of 2000 (64 a split) 9.4 / 10.3, of 6000 (192) 14.7 / 10.7; two splits
+//     that leave CUs idle (12 sequences) about equal from 2000 on.
 // (choose_split_tokens, the caller's choice of split sizes, mirrors it.)
 bool half_page_splits_pay(int64_t units, int64_t span, int64_t max_splits, int64_t D,
                           int64_t capacity) {
   const int64_t cus = lc_cu_count();
   if (max_splits == 1) {
     const int64_t round = cus * (D <= 64 ? 2 : 1), rounds = (units + round - 1) / round;
-    const int64_t tokens = (D <= 64 ? 48 : 80) * rounds;
-    return rounds <= 1 || span >= (tokens < 512 ? tokens : 512);
+    return rounds <= 1 || (rounds <= 3 && span >= (D <= 64 ? 48 : 80) * rounds);
   }
-  return capacity >= 896 && span >= 192 &&
+  return capacity >= 1792 && span >= 192 &&
          (max_splits > 2 || span >= 1024 || 8 * units * max_splits >= 7 * cus);
 }
 

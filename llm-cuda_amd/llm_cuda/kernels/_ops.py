@@ -904,8 +904,8 @@ def _half_page_splits_pay(units: int, span: int, max_splits: int, head_dim: int,
     if max_splits == 1:
         per_cu, tokens = (2, 48) if head_dim <= 64 else (1, 80)
         rounds = -(-units // (per_cu * n_cus))
-        return rounds <= 1 or span >= min(512, tokens * rounds)
-    return (capacity_tokens >= 896 and span >= 192
+        return rounds <= 1 or (rounds <= 3 and span >= tokens * rounds)
+    return (capacity_tokens >= 1792 and span >= 192
             and (max_splits > 2 or span >= 1024 or 8 * units * max_splits >= 7 * n_cus))
 
 

@@ -287,14 +287,15 @@ def test_split_heuristic_of_16_token_pages():
         return takes_workgroup_splits(batch * hkv, split, n, 16, d, cap), n
 
     # short contexts: a wave's share would be a step at most
-    for batch, tokens in ((1, 100), (3, 600), (1, 2000), (16, 600), (300, 100), (300, 400),
-                          (500, 300)):
+    # or many rounds of single splits, whose starts count where contexts are short
+    for batch, tokens in ((1, 100), (3, 600), (1, 2000), (16, 600), (8, 1000), (300, 100),
+                          (300, 400), (500, 300), (128, 400), (300, 600)):
         assert not route(batch, tokens)[0] and not route(batch, tokens, tokens)[0]
         cap = -(-tokens // 16) * 16
         assert (choose_split_tokens(batch, 8, 4, cap, 16)
                 == choose_split_tokens(batch, 8, 4, cap, 16, masked=True))
-    # a single split of at most a round of workgroups, and of more with more tokens
-    for batch, tokens in ((32, 100), (64, 300), (128, 400), (300, 600)):
+    # a single split of at most a round of workgroups, and of up to three with more tokens
+    for batch, tokens in ((32, 100), (64, 300), (90, 400), (96, 600)):
         assert route(batch, tokens) == (True, 1) == route(batch, tokens, tokens)
     assert route(64, 100, d=64) == (True, 1) and not route(96, 30, d=64)[0]
     # one round of the CUs whatever the lengths

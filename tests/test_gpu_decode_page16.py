@@ -53,7 +53,7 @@ def _reference(q, kp, vp, bt, sl):
 @pytest.mark.parametrize("lens,Hq,Hkv,D,dtype,bad,split", [
     ([0, 1, 15, 16, 17, 31, 32, 33], 8, 2, 128, torch.bfloat16, (), None),
     ([700, 513, 80], 8, 2, 64, torch.float16, ((0, 3), (0, 4), (1, 31)), 768),
-    ([1500, 1033, 80], 8, 2, 64, torch.float16, ((0, 3), (0, 40), (1, 64)), 192),
+    ([1900, 1033, 80], 8, 2, 64, torch.float16, ((0, 3), (0, 40), (1, 64)), 192),
     ([2500] + [100 * i + 7 for i in range(39)], 32, 8, 128, torch.bfloat16, ((5, 0),), None),
     ([300, 47], 40, 2, 256, torch.float16, (), 320),   # two head groups
     ([2047, 900], 4, 1, 96, torch.bfloat16, ((0, 127),), 256),
