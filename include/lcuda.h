@@ -334,6 +334,8 @@ LC_API int64_t lc_paged_decode_counter_count(void);
  * split_tokens: tokens per split (multiple of 64); max_splits *
  *   split_tokens must cover the block-table capacity max_pages_per_seq *
  *   page_size (so no clamped length can need more splits than the grid has).
+ *   On 16-token pages a grid of one workgroup per split and at most one per CU
+ *   cuts each sequence into up to max_splits equal parts of its own length.
  *   max_splits == 1 (bf16/f16, page_size a multiple of 32, a capacity within
  *   the limit of lc_paged_decode_step) runs one workgroup of 8 waves (4 above
  *   head_dim 128) per (sequence, head group) that shares the sequence's

@@ -954,7 +954,7 @@ def choose_split_tokens(batch: int, n_kv_heads: int, group: int, capacity_tokens
     would touch over 64 pages, and three things differ: fewer units than CUs make
     one round whatever the lengths (3 sequences of 6000 tokens at 8 kv heads: 17.4
     us in one round, 25.1 as the 90% rule's 19 splits each); ragged batches of
-    over two rounds of units within 4096 tokens are not split (96 of up to 3000 at
+    over 512 units within 4096 tokens are not split (96 of up to 3000 at
     D 64: 58 us, 76 at 2048-token splits, 70 in one-wave splits); ragged batches of
     head_dims that the tiles pad (not 64 or 128) stay in one-wave splits (D 256, 2 kv
     heads, 96 of up to 1200: 32 us, 44 in workgroups). Where the library would run such a split size
